@@ -1,0 +1,357 @@
+// Batched Q8_0 GEMM of many tokens on gfx950: 32 x 32 MFMA tiles.
+//
+// The result is the GEMV's (fkv_gemv.hip) bit for bit: per output, starting from +0 and
+// for each 32-value block in order, acc += f32(sumi) * (w_scale * x_scale)
+// (crates/kernels/src/q8_dot.rs:72-109), the product and the sum each rounded once.
+//
+// What bounds it: one v_mfma_i32_32x32x32_i8 (32 cycles) gives a block's integer dots of
+// 1,024 outputs, and then the VALU has to round and add each output by itself, 16 a lane.
+// So every instruction per output counts. Written as in the reference there are four
+// (convert, the product of the scales, the product, the sum); here three:
+// - the accumulator input of the integer MFMA is the bit pattern of M = 1.5 * 2^23, so
+//   its result, read as an f32, is M + sumi exactly (|sumi| <= 32 * 128 * 128 < 2^22),
+//   and one subtraction (exact; 2 a 4-cycle slot from two waves, a v_cvt_f32_i32 only
+//   one) gives f32(sumi);
+// - w_scale * x_scale of 1,024 outputs and two blocks is one v_mfma_f32_32x32x4_2b_f16
+//   whose second to fourth terms are zero: the product of two binary16 values is exact in
+//   f32, Inf and NaN included. (The f32 form of the same outer product held up the VALU:
+//   780 against 953 TFLOP/s in a register-only loop of these instructions.)
+// Measured at 512 tokens on Llama-3-8B's projections (one box, with the quantizer; before:
+// 16 x 16 tiles, one a wave, on the four-instruction epilogue): q/k/v 85.7 -> 55.0 us,
+// attn_output 55.1 -> 40.4, gate/up 344 -> 249 (483 TFLOP/s), down 171 -> 125. Three waves
+// a SIMD take 217 cycles a block together; the clock is 1.6-1.8 GHz under that load.
+#include "fkv_device.h"
+#include "fkv_q8_act.h"
+
+namespace fkv {
+namespace {
+
+typedef float f32x4a __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t u32x4a __attribute__((ext_vector_type(4), aligned(4)));
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+typedef int i32x16 __attribute__((ext_vector_type(16)));
+typedef int i32x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x32 __attribute__((ext_vector_type(32)));
+
+constexpr uint32_t kQ8Bytes = 34;
+[[maybe_unused]] constexpr uint32_t kPairBytes = 2 * kQ8Bytes;
+constexpr uint32_t kTileRows = 64;      // weight rows of a workgroup
+[[maybe_unused]] constexpr uint32_t kMagicBits = 0x4b400000u;
+[[maybe_unused]] constexpr float kMagic = 12582912.0f;    // 1.5 * 2^23
+
+// The activation in the workspace, per 16-token tile (tokens past n_tokens quantize to
+// zeros): a block's 512 bytes are 16-byte units (half of the block, token), blocks one
+// after the other; then, after every tile's quants, its scales, binary16 bits in 32,
+// [block][token]. An even block's quants are in the order its weights are read in (Chunk):
+// 0, 1, 30, 31, then 2 .. 29.
+__host__ __device__ constexpr uint64_t act_quant_bytes(uint32_t n_tiles, uint32_t nb) {
+  return (uint64_t)n_tiles * nb * 512u;
+}
+
+constexpr uint32_t kActThreads = 64;
+
+__global__ __launch_bounds__(kActThreads) void q8_act_tile_kernel(const float* __restrict__ x,
+                                                                  uint32_t cols, uint32_t n_tokens,
+                                                                  uint32_t n_tiles,
+                                                                  uint8_t* __restrict__ ws) {
+  // Item i: token t = i / (cols/8), values 8j .. 8j + 7 with j = i % (cols/8): quarter
+  // j % 4 of block j / 4, so a quad of lanes holds a block.
+  const uint32_t per = cols / 8u, nb = cols / 32u;
+  const uint64_t i = (uint64_t)blockIdx.x * kActThreads + threadIdx.x;
+  if (i >= (uint64_t)n_tiles * 16u * per) return;
+  const uint32_t t = (uint32_t)(i / per), j = (uint32_t)(i % per);
+  f32x4a a = {0.0f, 0.0f, 0.0f, 0.0f}, b = {0.0f, 0.0f, 0.0f, 0.0f};
+  if (t < n_tokens) {
+    const float* src = x + (uint64_t)t * cols + 8u * j;
+    a = *(const f32x4a*)src;
+    b = *(const f32x4a*)(src + 4);
+  }
+  float m = __builtin_fmaxf(__builtin_fabsf(a.x), __builtin_fabsf(a.y));
+  m = __builtin_fmaxf(m, __builtin_fabsf(a.z));
+  m = __builtin_fmaxf(m, __builtin_fabsf(a.w));
+  m = __builtin_fmaxf(m, __builtin_fabsf(b.x));
+  m = __builtin_fmaxf(m, __builtin_fabsf(b.y));
+  m = __builtin_fmaxf(m, __builtin_fabsf(b.z));
+  m = __builtin_fmaxf(m, __builtin_fabsf(b.w));
+  m = __builtin_fmaxf(m, 0.0f);  // all NaN: 0, as the reference's amax = 0 start
+  m = __builtin_fmaxf(m, dev::dpp<0xB1>(m));
+  m = __builtin_fmaxf(m, dev::dpp<0x4E>(m));
+  const float d = dev::div127(m);
+  const float id = (d != 0.0f) ? 1.0f / d : 0.0f;
+  const uint32_t qa = dev::q8_byte(a.x * id) | (dev::q8_byte(a.y * id) << 8) |
+                      (dev::q8_byte(a.z * id) << 16) | (dev::q8_byte(a.w * id) << 24);
+  const uint32_t qb = dev::q8_byte(b.x * id) | (dev::q8_byte(b.y * id) << 8) |
+                      (dev::q8_byte(b.z * id) << 16) | (dev::q8_byte(b.w * id) << 24);
+  const uint32_t tt = t / 16u, c = t % 16u, blk = j / 4u, quarter = j % 4u;
+  const uint64_t at = (uint64_t)tt * nb + blk;
+  uint32_t lo = qa, hi = qb;
+  if (blk % 2u == 0u) {
+    // quads rotate: the lane before (the last one's for the first) holds 2 of these bytes
+    const uint32_t prev = (uint32_t)__builtin_amdgcn_mov_dpp((int)qb, 0x93, 0xf, 0xf, true);
+    lo = quarter == 0u ? (qa & 0xffffu) | (prev & 0xffff0000u) : __builtin_amdgcn_alignbit(qa, prev, 16);
+    hi = __builtin_amdgcn_alignbit(qb, qa, 16);
+  }
+  *(uint2*)(ws + at * 512u + (quarter / 2u) * 256u + c * 16u + (quarter % 2u) * 8u) =
+      make_uint2(lo, hi);
+  if (quarter == 0u)
+    ((uint32_t*)(ws + act_quant_bytes(n_tiles, nb)))[at * 16u + c] = dev::f16_bits_away(d);
+}
+
+// A chunk of 4 blocks (2 pairs) in LDS. A pair of a weight row is 17 dwords, [scale 0 |
+// quants 0, 1] [2 .. 5] ... [26 .. 29] [30, 31 | scale 1] and 8 of the odd block's quants:
+// as 16-byte units, dwords 0-3, 4-7, 9-12 and 13-16, and dword 8 by itself. The units of
+// the odd block are its quants; the even block's are too, but for dword 0, which with
+// dword 8 gives quants 0, 1, 30, 31 (one v_perm, a second one the scales): a dot does not
+// depend on the order of its terms, so nothing is realigned.
+// A row's units lie at unit ^ (row / 4) % 4: a wave stages 16 rows' with one load (4 lanes
+// a row, 64 consecutive bytes) and reads one unit of 32 rows, both over all banks.
+struct Chunk {
+  uint4 wq[2][kTileRows][4];   // [pair][row][unit, at unit ^ (row / 4) % 4]
+  uint4 xq[2][4][2][32];       // [token half][block][half of the block][token]
+  uint32_t we[2][kTileRows];   // [pair][row]
+  uint32_t xs[2][2][2][32];    // [pair][token half][block][token]
+};
+
+// A workgroup: 64 weight rows x 64 tokens, a wave 32 x 32; 3 workgroups a CU (157 VGPRs,
+// 52.5 KiB of LDS). Everything is staged by loads straight into LDS, two to three chunks
+// ahead (three buffers), so that no wave spends registers or instructions on it. (Weights
+// through registers with the repacking done by the computing waves: gate/up 285 us; by two
+// or four further waves: 264-300.)
+// Tokens are the MFMA rows and weight rows its columns, so a lane's results are one
+// column of y and 32 consecutive lanes store 128 consecutive bytes.
+__global__ __launch_bounds__(256, 2) void gemm_q8_tile_kernel(const GemvBatch bat, uint32_t cols,
+                                                              uint32_t n_tokens, uint32_t n_tiles,
+                                                              uint32_t row_tiles,
+                                                              uint32_t token_tiles,
+                                                              const uint8_t* __restrict__ ws) {
+#ifdef __HIP_DEVICE_COMPILE__  // the host pass needs the kernel's stub only
+  // Workgroups are dealt to the 8 XCDs in turn; the token tiles of one row tile follow
+  // each other on one XCD, whose L2 then reads the weights once.
+  const uint32_t xcd = blockIdx.x % 8u, j8 = blockIdx.x / 8u;
+  const uint32_t rt = (j8 / token_tiles) * 8u + xcd, ty = j8 % token_tiles;
+  if (rt >= row_tiles) return;
+  uint32_t mi = 0;
+#pragma unroll
+  for (int j = 1; j < kGemvMaxMats; ++j)
+    if ((uint32_t)j < bat.n && rt >= bat.m[j].wg0) mi = (uint32_t)j;
+  const GemvMat M = mi == 0u ? bat.m[0] : mi == 1u ? bat.m[1] : mi == 2u ? bat.m[2] : bat.m[3];
+  const uint32_t rows = M.rows, row0 = (rt - M.wg0) * kTileRows;
+  const uint32_t nb = cols / 32u, np = nb / 2u, nc = (np + 1u) / 2u;
+  const uint32_t tid = threadIdx.x, lane = tid & 63u;
+  const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
+  const uint32_t c32 = lane & 31u, half = lane >> 5;
+  const uint32_t wr = wave & 1u, wt = wave >> 1;
+
+  __shared__ Chunk s0, s1, s2;
+
+  // Staging: loads straight into LDS, 6 a wave and chunk. Rows past the matrix, tokens
+  // past the batch and pairs past the row's end read the last one (never used).
+  const uint64_t row_bytes = (uint64_t)nb * kQ8Bytes;
+  const uint32_t last_row = rows - 1u - row0;
+  const uint32_t t16 = ty * 4u;
+  auto rsrc = [](const void* p) {
+    return __builtin_amdgcn_make_buffer_rsrc((void*)p, (short)0, 0x7fffffff, 0x00020000);
+  };
+  const __amdgpu_buffer_rsrc_t rw = rsrc(M.w + row0 * row_bytes);
+  const __amdgpu_buffer_rsrc_t rq = rsrc(ws + (uint64_t)t16 * nb * 512u);
+  const __amdgpu_buffer_rsrc_t rs = rsrc(ws + act_quant_bytes(n_tiles, nb) + (uint64_t)t16 * nb * 64u);
+  auto row_at = [&](uint32_t r) { return (r < last_row ? r : last_row) * (uint32_t)row_bytes; };
+  auto tile_at = [&](uint32_t j) { return t16 + j < n_tiles ? j : n_tiles - 1u - t16; };
+  // weights: wave w stages rows 16w .. 16w + 15, 4 lanes a row
+  const uint32_t unit = (lane & 3u) ^ (lane >> 4);
+  const uint32_t w_off = row_at(16u * wave + lane / 4u) + unit * 16u + (unit >= 2u ? 4u : 0u);
+  // their dwords 8: waves w and w + 2 pair w (the same ones), a lane a row
+  const uint32_t e_off = row_at(lane) + 32u;
+  // activation: wave w blocks 2 * (w / 2), + 1 of token half w % 2, and their scales
+  const uint32_t x_tile = tile_at(2u * (wave & 1u) + c32 / 16u) * nb;
+  const uint32_t xq_off = x_tile * 512u + half * 256u + (c32 % 16u) * 16u;
+  const uint32_t xs_off = x_tile * 64u + (c32 % 16u) * 4u;
+#define FKV_LDS(p) (__attribute__((address_space(3))) void*)(p)
+  auto stage = [&](uint32_t k, Chunk& L) __attribute__((always_inline)) {
+#pragma unroll
+    for (uint32_t i = 0; i < 2u; ++i) {
+      const uint32_t p = 2u * k + i < np ? 2u * k + i : np - 1u;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, FKV_LDS(&L.wq[i][16u * wave][0]), 16, w_off,
+                                               (int)(p * kPairBytes), 0, 0);
+      const uint32_t xb = 2u * (wave >> 1) + i, b = 4u * k + xb;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rq, FKV_LDS(&L.xq[wave & 1u][xb][0][0]), 16, xq_off,
+                                               (int)((b < nb ? b : nb - 1u) * 512u), 0, 0);
+    }
+    const uint32_t pe = wave & 1u, p = 2u * k + pe < np ? 2u * k + pe : np - 1u;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, FKV_LDS(&L.we[pe][0]), 4, e_off,
+                                             (int)(p * kPairBytes), 0, 0);
+    const uint32_t b = 4u * k + 2u * (wave >> 1) + half;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, FKV_LDS(&L.xs[wave >> 1][wave & 1u][0][0]), 4,
+                                             xs_off + (b < nb ? b : nb - 1u) * 64u, 0, 0, 0);
+  };
+#undef FKV_LDS
+  // This wave's reads of the chunk to be overwritten are done, and its loads of the next
+  // chunk have landed (those of the chunk after it, the last 6, may still be in flight);
+  // then every wave's.
+  auto sync = [&]() __attribute__((always_inline)) {
+    __asm__ volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0x0076);  // vmcnt(6) lgkmcnt(0)
+    __builtin_amdgcn_s_barrier();
+    __asm__ volatile("" ::: "memory");
+  };
+
+  float acc[16];
+#pragma unroll
+  for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+  i32x16 magic;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) magic[r] = (int)kMagicBits;
+  __asm__("" : "+v"(magic));  // kept in registers: not written anew for every product
+
+  // A pair's operands, and its products: the integer dots of its blocks and both blocks'
+  // products of scales.
+  i32x2 w1 = {0, 0}, x1 = {0, 0};
+  i32x4 wq0, wq1, xq0, xq1;
+  uint32_t we;
+  f32x32 P;
+  i32x16 D0, D1;
+  const f32x32 zero = {};
+  const uint32_t row_l = wr * 32u + c32, u0 = half ^ (c32 / 4u) % 4u;
+  // v_perm selectors of the even block's first dword (lanes 0-31: quants 0, 1, 30, 31;
+  // the others' is as stored) and of the scale (lanes 0-31 the even block's)
+  const uint32_t sel_q = half ? 0x03020100u : 0x05040302u, sel_s = half ? 0x0c0c0706u : 0x0c0c0100u;
+  auto read_0 = [&](const Chunk& L, int s) __attribute__((always_inline)) {
+    wq0 = __builtin_bit_cast(i32x4, L.wq[s][row_l][u0]);
+    we = L.we[s][row_l];
+    xq0 = __builtin_bit_cast(i32x4, L.xq[wt][2 * s][half][c32]);
+    x1[0] = (int)L.xs[s][wt][half][c32];
+  };
+  auto read_1 = [&](const Chunk& L, int s) __attribute__((always_inline)) {
+    wq1 = __builtin_bit_cast(i32x4, L.wq[s][row_l][u0 ^ 2u]);
+    xq1 = __builtin_bit_cast(i32x4, L.xq[wt][2 * s + 1][half][c32]);
+  };
+  auto dots_0 = [&]() __attribute__((always_inline)) {
+    w1[0] = (int)__builtin_amdgcn_perm(we, (uint32_t)wq0[0], sel_s);
+    wq0[0] = (int)__builtin_amdgcn_perm(we, (uint32_t)wq0[0], sel_q);
+    D0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(xq0, wq0, magic, 0, 0, 0);
+  };
+  auto scales = [&]() __attribute__((always_inline)) {
+    P = __builtin_amdgcn_mfma_f32_32x32x4f16(__builtin_bit_cast(f16x4, x1),
+                                             __builtin_bit_cast(f16x4, w1), zero, 0, 0, 0);
+  };
+  auto sub16 = [&](f32x16& f) __attribute__((always_inline)) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) f[r] = f[r] - kMagic;
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto mul16 = [&](f32x16& f, int o) __attribute__((always_inline)) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) f[r] = f[r] * P[o + r];
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto add16 = [&](float (&a)[16], const f32x16& f) __attribute__((always_inline)) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) a[r] = a[r] + f[r];
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // A pair from P, D0, D1; each is replaced by the next pair's as soon as it is used up,
+  // from the operands in registers, which are then read anew for the pair after that
+  // (pair s of L). What an MFMA writes is used 32 to 64 instructions later.
+  auto pair = [&](const Chunk& L, int s, auto between) __attribute__((always_inline)) {
+    f32x16 f = __builtin_bit_cast(f32x16, D0);
+    sub16(f);
+    mul16(f, 0);
+    add16(acc, f);
+    dots_0();
+    __builtin_amdgcn_sched_barrier(0);
+    f = __builtin_bit_cast(f32x16, D1);
+    sub16(f);
+    mul16(f, 16);
+    scales();
+    __builtin_amdgcn_sched_barrier(0);
+    between();
+    read_0(L, s);
+    __builtin_amdgcn_sched_barrier(0);
+    add16(acc, f);
+    D1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(xq1, wq1, magic, 0, 0, 0);
+    read_1(L, s);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // Chunk k while chunk k + 1 (N) is read and chunk k + 3 staged into L, whose reads all
+  // waves have finished.
+  auto chunk = [&](Chunk& L, Chunk& N, uint32_t k) __attribute__((always_inline)) {
+    pair(N, 0, [&]() __attribute__((always_inline)) {
+      sync();
+      stage(k + 3u, L);
+    });
+    if (2u * k + 1u < np) pair(N, 1, [] {});
+  };
+
+  stage(0, s0);
+  stage(1, s1);
+  sync();
+  stage(2, s2);
+  read_0(s0, 0);
+  read_1(s0, 0);
+  dots_0();
+  scales();
+  D1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(xq1, wq1, magic, 0, 0, 0);
+  read_0(s0, 1);
+  read_1(s0, 1);
+  for (uint32_t k = 0;; k += 3u) {
+    chunk(s0, s1, k);
+    if (k + 1u >= nc) break;
+    chunk(s1, s2, k + 1u);
+    if (k + 2u >= nc) break;
+    chunk(s2, s0, k + 2u);
+    if (k + 3u >= nc) break;
+  }
+  __builtin_amdgcn_s_waitcnt(0x0f70);  // no load into LDS outlives the workgroup
+
+  const uint32_t row = row0 + wr * 32u + c32;
+  if (row >= rows) return;
+  const uint32_t tok0 = (ty * 2u + wt) * 32u + 4u * half;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    const uint32_t tok = tok0 + 8u * (uint32_t)(r / 4) + (uint32_t)(r % 4);
+    if (tok < n_tokens) M.y[(uint64_t)tok * rows + row] = acc[r];
+  }
+#endif
+}
+
+}  // namespace
+
+// A workgroup takes about as long alone on its CU as with two others (4,096 columns: 25 us
+// at one a CU, 34 us at three), so the kernel wins once every CU has one: at 256
+// workgroups and 4,096 x 4,096 weights 28.1 us against 30.5 for the 16 x 16 kernel (256
+// tokens), at 192 27.0 against 24.3 (192 tokens); 2,048 and 14,336 columns turn at the same
+// count (17.4 / 19.4 and 77.5 / 85.7 us at 256). And the tokens have to fill most of its 64:
+// 28,672 rows, 32 tokens 48.5 us against 44.4, 64 tokens 50.7 against 55.5.
+constexpr uint64_t kTileMinWgs = 256;
+constexpr uint32_t kTileMinTokens = 48;
+bool gemm_tile_fills(const GemvBatch& b, uint32_t n_tokens) {
+  uint64_t row_tiles = 0;
+  for (uint32_t m = 0; m < b.n; ++m) row_tiles += (b.m[m].rows + kTileRows - 1u) / kTileRows;
+  const uint64_t wgs = row_tiles * ((n_tokens + 63u) / 64u);
+  return n_tokens >= kTileMinTokens && wgs >= kTileMinWgs && wgs < (1ull << 30);
+}
+
+hipError_t launch_gemm_q8_tile(GemvBatch b, uint32_t cols, const float* x, uint32_t n_tokens,
+                               void* workspace, hipStream_t s) {
+  uint32_t row_tiles = 0;
+  for (uint32_t m = 0; m < b.n; ++m) {
+    b.m[m].wg0 = row_tiles;
+    row_tiles += (b.m[m].rows + kTileRows - 1u) / kTileRows;
+  }
+  for (uint32_t m = b.n; m < (uint32_t)kGemvMaxMats; ++m) b.m[m] = b.m[0];
+  const uint32_t n_tiles = (n_tokens + 15u) / 16u;
+  const uint64_t items = (uint64_t)n_tiles * 16u * (cols / 8u);
+  q8_act_tile_kernel<<<(uint32_t)((items + kActThreads - 1u) / kActThreads), kActThreads, 0, s>>>(
+      x, cols, n_tokens, n_tiles, (uint8_t*)workspace);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  const uint32_t token_tiles = (n_tiles + 3u) / 4u;
+  const uint32_t grid = (row_tiles + 7u) / 8u * 8u * token_tiles;
+  gemm_q8_tile_kernel<<<grid, 256, 0, s>>>(b, cols, n_tokens, n_tiles, row_tiles, token_tiles,
+                                           (const uint8_t*)workspace);
+  return hipGetLastError();
+}
+
+}  // namespace fkv

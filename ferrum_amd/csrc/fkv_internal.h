@@ -275,5 +275,10 @@ bool gemm_mfma_eligible(const GemvBatch& b, uint32_t cols, uint32_t n_tokens);
 uint64_t gemm_mfma_workspace_bytes(uint32_t cols, uint32_t n_tokens);
 hipError_t launch_gemm_q8_mfma(GemvBatch b, uint32_t cols, const float* x, uint32_t n_tokens,
                                void* workspace, hipStream_t s);
+// The same in 32 x 32 tiles for many tokens (fkv_gemm.hip), with the same workspace, and
+// whether a launch is large enough for it. cols % 64 == 0, weights 4-byte aligned.
+bool gemm_tile_fills(const GemvBatch& b, uint32_t n_tokens);
+hipError_t launch_gemm_q8_tile(GemvBatch b, uint32_t cols, const float* x, uint32_t n_tokens,
+                               void* workspace, hipStream_t s);
 
 }  // namespace fkv

@@ -110,6 +110,24 @@ def test_non_finite_and_extreme_inputs():
     _same(got, want)
 
 
+@pytest.mark.parametrize("rows,cols,n_tokens", [
+    ([16385], 1024, 48),              # the fewest tokens, one row past the last row tile
+    ([8200], 2048, 65),               # one token past a tile
+    ([4032, 64, 1], 1024, 256),       # three matrices, whole tiles and one row
+    ([4100], 3072, 250),
+])
+def test_large_launches_in_32x32_tiles(rows, cols, n_tokens):
+    """Launches of 256 workgroups of 64 x 64 outputs or more, non-finite scales among the
+    weights and activations: every output is the oracle's."""
+    rng = np.random.default_rng(cols + n_tokens)
+    ws = [_weights(rng, r, cols, special=True) for r in rows]
+    x = (rng.standard_normal((n_tokens, cols)) *
+         rng.choice([1e-4, 1.0, 300.0], (n_tokens, 1))).astype(np.float32)
+    x[1, 70], x[2, 100], x[3, 3], x[4, 32:64] = np.inf, -np.inf, np.nan, 3e38
+    for r, w, y in zip(rows, ws, _batched(ws, rows, cols, x)):
+        _same(y, ref.q8_gemm(w, r, cols, x))
+
+
 @pytest.mark.parametrize("rows,cols,n_tokens,offset", [
     (20, 1024, 7, 0),    # too few tokens: GEMV
     (20, 544, 30, 0),    # columns off a multiple of 1024: GEMV
