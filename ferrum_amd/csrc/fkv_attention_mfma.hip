@@ -2322,8 +2322,12 @@ __global__ void __launch_bounds__(256) pf_stage_q8_kernel(
 // Merges the key-range pieces of every prefill workgroup cut into more than one:
 // out = sum_z 2^(m_z - M) o_z / sum_z 2^(m_z - M) l_z with M = max_z m_z (0 where M is
 // not finite, as the single-piece path writes). Grid (n_seqs * n_kv_heads, tile
-// groups): one workgroup per prefill workgroup, thread t on dim t % D of columns
-// t / D, t / D + 256 / D, ...
+// groups, column groups): a thread takes 4 dims of one column, so a workgroup's 256 / (D / 4)
+// columns are merged at once and a launch has that many times the waves. The kernel is
+// bound by the latency of a column's few dependent loads (a piece's 32 KiB come from L2 or
+// the memory-side cache): one workgroup going through its 64 columns 2 at a time took 46.1
+// us where the attention before it took 41.9 (one 389-token chunk behind 2,011 tokens,
+// Llama-3-8B heads, 3 pieces).
 template <int D>
 __global__ void __launch_bounds__(256) attn_prefill_combine_kernel(
     uint32_t n_kv_heads, uint32_t n_heads, uint32_t G, uint32_t max_blocks,
@@ -2340,28 +2344,39 @@ __global__ void __launch_bounds__(256) attn_prefill_combine_kernel(
   const int32_t npiece = pf_pieces(pf_wg_blocks(sq, tile0, T), split_blocks, max_splits);
   if (npiece <= 1) return;
   const uint64_t slot0 = ((uint64_t)sk * gridDim.y + blockIdx.y) * max_splits;
-  constexpr uint32_t kCols = kAttnWaves * 16, kStride = 256 / D;
-  const uint32_t d = threadIdx.x % D;
-  const int64_t qrow0 = q_offsets[seq];
-  for (uint32_t cc = threadIdx.x / D; cc < kCols; cc += kStride) {
-    const int32_t c = (int32_t)(cc % 16u);
-    const int32_t jc = (tile0 + (int32_t)(cc / 16u)) * T + c / (int32_t)G;
-    if (c >= T * (int32_t)G || jc >= sq.ql) continue;
-    float M = -__builtin_inff();
-    for (int32_t z = 0; z < npiece; z++)
-      M = __builtin_fmaxf(M, ws_ml[((slot0 + z) * kCols + cc) * 2]);
-    float o = 0.0f, L = 0.0f;
-    if (__builtin_isfinite(M)) {
-      for (int32_t z = 0; z < npiece; z++) {
-        const uint64_t i = (slot0 + z) * kCols + cc;
-        const float w = __builtin_amdgcn_exp2f(ws_ml[i * 2] - M);
-        o = __builtin_fmaf(w, ws_o[i * D + d], o);
-        L = __builtin_fmaf(w, ws_ml[i * 2 + 1], L);
-      }
+  constexpr uint32_t kCols = kAttnWaves * 16, kLanes = D / 4;
+  const uint32_t d = threadIdx.x % kLanes * 4u;
+  const uint32_t cc = blockIdx.z * (256u / kLanes) + threadIdx.x / kLanes;
+  const int32_t c = (int32_t)(cc % 16u);
+  const int32_t jc = (tile0 + (int32_t)(cc / 16u)) * T + c / (int32_t)G;
+  if (c >= T * (int32_t)G || jc >= sq.ql) return;
+  const float* ml = ws_ml + (slot0 * kCols + cc) * 2;
+  const float* po = ws_o + (slot0 * kCols + cc) * D + d;
+  float M = -__builtin_inff();
+#pragma unroll 4
+  for (int32_t z = 0; z < npiece; z++) M = __builtin_fmaxf(M, ml[(uint64_t)z * kCols * 2]);
+  float4 o = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  float L = 0.0f;
+  const bool fin = __builtin_isfinite(M);
+  if (fin) {
+#pragma unroll 4
+    for (int32_t z = 0; z < npiece; z++) {
+      const float w = __builtin_amdgcn_exp2f(ml[(uint64_t)z * kCols * 2] - M);
+      const float4 v = *(const float4*)(po + (uint64_t)z * kCols * D);
+      o.x = __builtin_fmaf(w, v.x, o.x);
+      o.y = __builtin_fmaf(w, v.y, o.y);
+      o.z = __builtin_fmaf(w, v.z, o.z);
+      o.w = __builtin_fmaf(w, v.w, o.w);
+      L = __builtin_fmaf(w, ml[(uint64_t)z * kCols * 2 + 1], L);
     }
-    const uint64_t row = ((uint64_t)(qrow0 + jc) * n_heads + (uint64_t)kvh * G + (uint64_t)(c % (int32_t)G)) * D;
-    out[row + d] = __builtin_isfinite(M) ? o * (1.0f / L) : 0.0f;
   }
+  const uint64_t row = ((uint64_t)(q_offsets[seq] + jc) * n_heads + (uint64_t)kvh * G + (uint64_t)(c % (int32_t)G)) * D;
+  const float r = fin ? 1.0f / L : 0.0f;
+  float* dst = out + row + d;  // 4-byte stores: out has a float's alignment
+  dst[0] = fin ? o.x * r : 0.0f;
+  dst[1] = fin ? o.y * r : 0.0f;
+  dst[2] = fin ? o.z * r : 0.0f;
+  dst[3] = fin ? o.w * r : 0.0f;
 }
 
 // Workgroups of the stream kernel one CU holds at once (0 if it cannot launch).
@@ -2558,7 +2573,8 @@ hipError_t launch_prefill_attention(const Geom& g, uint32_t layer, uint32_t n_he
   e = hipGetLastError();
   if (e != hipSuccess || !split) return e;
   // the combine reads the table width only as the context cap
-  const dim3 cgrid(n_seqs * g.n_kv_heads, plan.tile_groups);
+  const dim3 cgrid(n_seqs * g.n_kv_heads, plan.tile_groups,
+                   (uint32_t)(kAttnWaves * 16) * (g.head_dim / 4u) / 256u);
   if (g.head_dim == 128)
     attn_prefill_combine_kernel<128><<<cgrid, 256, 0, s>>>(g.n_kv_heads, n_heads, G, cap_blocks,
                                                            ctx_lens, q_lens, q_offsets, max_q_len,
