@@ -1492,7 +1492,7 @@ int32_t fkv_gemm_q8_0_batched_workspace_size(uint64_t cols, uint64_t n_tokens,
                                              uint64_t* bytes_out) {
   if (!bytes_out) return fail(FKV_ERR_INVALID, "null argument");
   *bytes_out = 0;
-  if (cols == 0 || cols % 1024 != 0 || cols > 0xffffffffull || n_tokens > 0x7fff0000ull ||
+  if (cols == 0 || cols % 64 != 0 || cols > 0xffffffffull || n_tokens > 0x7fff0000ull ||
       n_tokens < fkv::kGemmMfmaMinTokens)
     return ok();  // such calls run the GEMV and need no workspace
   *bytes_out = fkv::gemm_mfma_workspace_bytes((uint32_t)cols, (uint32_t)n_tokens);
@@ -1508,15 +1508,19 @@ int32_t fkv_gemm_q8_0_batched(uint32_t n_mats, const void* const* w, const uint6
   int32_t st = gemm_q8_batch(n_mats, w, w_len, rows, cols, x, x_len, n_tokens, y, y_len, &b);
   if (st) return st;
   if (b.n == 0) return ok();
-  if (!fkv::gemm_mfma_eligible(b, (uint32_t)cols, (uint32_t)n_tokens)) {
+  const bool eligible = fkv::gemm_mfma_eligible(b, (uint32_t)cols, (uint32_t)n_tokens);
+  const uint64_t need =
+      eligible ? fkv::gemm_mfma_workspace_bytes((uint32_t)cols, (uint32_t)n_tokens) : 0;
+  const bool small = !workspace || workspace_bytes < need;
+  const bool aligned = (uintptr_t)workspace % 16 == 0;
+  if (eligible && (small || !aligned) && fkv::gemm_mfma_needs_workspace(b, (uint32_t)cols))
+    return fail(FKV_ERR_INVALID,
+                small ? "gemm workspace too small" : "gemm workspace must be 16-byte aligned");
+  if (!eligible || small || !aligned) {
     FKV_HIP(fkv::launch_gemv_q8(b, (uint32_t)cols, x, (uint32_t)n_tokens, (hipStream_t)stream),
             "gemv launch");
     return ok();
   }
-  const uint64_t need = fkv::gemm_mfma_workspace_bytes((uint32_t)cols, (uint32_t)n_tokens);
-  if (!workspace || workspace_bytes < need) return fail(FKV_ERR_INVALID, "gemm workspace too small");
-  if ((uintptr_t)workspace % 16 != 0)
-    return fail(FKV_ERR_INVALID, "gemm workspace must be 16-byte aligned");
   FKV_HIP(fkv::launch_gemm_q8_mfma(b, (uint32_t)cols, x, (uint32_t)n_tokens, workspace,
                                    (hipStream_t)stream),
           "gemm launch");

@@ -1,4 +1,7 @@
-// Batched Q8_0 GEMM of many tokens on gfx950: 32 x 32 MFMA tiles.
+// Batched Q8_0 GEMM on the matrix cores of gfx950, for batches of activation rows (a
+// decode step's sequences, a prefill chunk): the GEMV reads every weight once per 4
+// tokens. The activation is quantized once, into a workspace; then one of two kernels,
+// 32 x 32 tiles first.
 //
 // The result is the GEMV's (fkv_gemv.hip) bit for bit: per output, starting from +0 and
 // for each 32-value block in order, acc += f32(sumi) * (w_scale * x_scale)
@@ -42,16 +45,18 @@ constexpr uint32_t kTileRows = 64;      // weight rows of a workgroup
 [[maybe_unused]] constexpr float kMagic = 12582912.0f;    // 1.5 * 2^23
 
 // The activation in the workspace, per 16-token tile (tokens past n_tokens quantize to
-// zeros): a block's 512 bytes are 16-byte units (half of the block, token), blocks one
-// after the other; then, after every tile's quants, its scales, binary16 bits in 32,
-// [block][token]. An even block's quants are in the order its weights are read in (Chunk):
-// 0, 1, 30, 31, then 2 .. 29.
+// zeros): 512 bytes a block of quants in 16-byte units, then, after every tile's quants,
+// the scales, binary16 bits in 32, [tile][block][token]. An even block's quants are in the
+// order its weights are read in (Chunk): 0, 1, 30, 31, then 2 .. 29. A unit, for the
+// 32 x 32 kernel, is (block, half of the block, token); for the 16 x 16 kernel (kPairs)
+// (pair of blocks, quarter, token): that quarter's 8 quants of both blocks.
 __host__ __device__ constexpr uint64_t act_quant_bytes(uint32_t n_tiles, uint32_t nb) {
   return (uint64_t)n_tiles * nb * 512u;
 }
 
 constexpr uint32_t kActThreads = 64;
 
+template <bool kPairs>
 __global__ __launch_bounds__(kActThreads) void q8_act_tile_kernel(const float* __restrict__ x,
                                                                   uint32_t cols, uint32_t n_tokens,
                                                                   uint32_t n_tiles,
@@ -93,8 +98,9 @@ __global__ __launch_bounds__(kActThreads) void q8_act_tile_kernel(const float* _
     lo = quarter == 0u ? (qa & 0xffffu) | (prev & 0xffff0000u) : __builtin_amdgcn_alignbit(qa, prev, 16);
     hi = __builtin_amdgcn_alignbit(qb, qa, 16);
   }
-  *(uint2*)(ws + at * 512u + (quarter / 2u) * 256u + c * 16u + (quarter % 2u) * 8u) =
-      make_uint2(lo, hi);
+  const uint64_t to = kPairs ? (at - blk % 2u) * 512u + (quarter * 16u + c) * 16u + (blk % 2u) * 8u
+                             : at * 512u + (quarter / 2u) * 256u + c * 16u + (quarter % 2u) * 8u;
+  *(uint2*)(ws + to) = make_uint2(lo, hi);
   if (quarter == 0u)
     ((uint32_t*)(ws + act_quant_bytes(n_tiles, nb)))[at * 16u + c] = dev::f16_bits_away(d);
 }
@@ -316,41 +322,328 @@ __global__ __launch_bounds__(256, 2) void gemm_q8_tile_kernel(const GemvBatch ba
 #endif
 }
 
+// ---------------------------------------------------------------------------
+// Few workgroups of 64 x 64: 16 weight rows x 64 tokens a workgroup, 16 x 16 a wave.
+// ---------------------------------------------------------------------------
+//
+// The same sums (integer dots from v_mfma_i32_16x16x32_i8, four blocks' products of scales
+// from one v_mfma_f32_16x16x4_4b_f16, three VALU instructions per output and block), for
+// launches that would leave CUs without work in 64 x 64 tiles, or most of their tokens
+// unused. The ordered sum makes a row tile one chain, a wave takes about 80-90 cycles a
+// block, and a CU has few waves: the chain bounds launches of few rows (down of
+// Llama-3-8B, 448 blocks: 25 us at 16 tokens where the weights alone stream in 10), and
+// what matters is that nothing else is waited for. A further wave streams the weights
+// through a ring of chunks in LDS by direct loads; the computing waves load the
+// activation, which the L2 holds, four groups of blocks ahead into registers. Loads retire
+// in order, so with the weight loads in the computing waves each activation load would
+// wait for HBM. A short ring of small chunks leaves room for 4 to 8 workgroups a CU and
+// little to fill before the first block: 3 chunks of 8 blocks against 6 of 16, us at 16
+// tokens: q/k/v 11.5 / 13.5, attn_output 10.5 / 11.5, gate/up 38.4 / 44.5, down 24.9 / 26.3.
+// Against the kernel before (one variant with and one without such a wave, weights
+// through registers, four VALU instructions): 16 tokens 14.9, 12.6, 39.8, 26.4; 64 tokens
+// q/k/v 18.4 -> 15.9, attn_output 13.6 -> 12.9, down 32.6 -> 31.8.
+[[maybe_unused]] constexpr uint32_t kRing = 3;
+[[maybe_unused]] constexpr uint32_t kGroup = 4;    // blocks of a step
+constexpr uint32_t kPairs = 4;    // pairs of blocks of a chunk
+[[maybe_unused]] constexpr int kGroups = 2;        // and its groups
+constexpr uint32_t kRowTile = 16;
+
+struct RowChunk {
+  uint4 wq[kPairs][kRowTile][4];   // as Chunk's
+  uint32_t we[kPairs][kRowTile];
+};
+
+// kTail: columns not a multiple of 512. The blocks that fill the row's last chunk up load
+// its last ones again and get scales of zero, so they add +0.
+// W computing waves, a 16-token tile each.
+template <int W, bool kTail>
+__global__ __launch_bounds__((W + 1) * 64, 4) void gemm_q8_rows_kernel(const GemvBatch bat, uint32_t cols,
+                                                              uint32_t n_tokens, uint32_t n_tiles,
+                                                              const uint8_t* __restrict__ ws) {
+#ifdef __HIP_DEVICE_COMPILE__  // the host pass needs the kernel's stub only
+  uint32_t mi = 0;
+#pragma unroll
+  for (int j = 1; j < kGemvMaxMats; ++j)
+    if ((uint32_t)j < bat.n && blockIdx.x >= bat.m[j].wg0) mi = (uint32_t)j;
+  const GemvMat M = mi == 0u ? bat.m[0] : mi == 1u ? bat.m[1] : mi == 2u ? bat.m[2] : bat.m[3];
+  const uint32_t rows = M.rows, row0 = (blockIdx.x - M.wg0) * kRowTile;
+  const uint32_t nb = cols / 32u, np = nb / 2u;
+  // groups, runs of 4 groups
+  const uint32_t ng = (nb + kGroup - 1u) / kGroup, n4 = (ng + 3u) / 4u;
+  // barriers: one a chunk, and two chunks read past the row's end (up to 3 groups ahead)
+  const uint32_t n_bar = 2u + n4 * 2u;
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const uint32_t c = lane & 15u, grp = lane >> 4;
+
+  __shared__ RowChunk ring[kRing];
+  auto barrier = [] {
+    __asm__ volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    __asm__ volatile("" ::: "memory");
+  };
+
+  if (wave == (uint32_t)W) {
+    // Rows past the matrix and pairs past the row's end load the last one (never used, or
+    // met by zero scales).
+    const uint64_t row_bytes = (uint64_t)nb * kQ8Bytes;
+    const uint32_t last_row = rows - 1u - row0;
+    const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(M.w + row0 * row_bytes), (short)0, 0x7fffffff, 0x00020000);
+    auto row_at = [&](uint32_t r) { return (r < last_row ? r : last_row) * (uint32_t)row_bytes; };
+    const uint32_t unit = (lane & 3u) ^ (lane >> 4);
+    const uint32_t w_off = row_at(lane / 4u) + unit * 16u + (unit >= 2u ? 4u : 0u);
+    const uint32_t e_off = row_at(c) + 32u;
+    auto stage = [&](uint32_t k) __attribute__((always_inline)) {
+      RowChunk& L = ring[k % kRing];
+#pragma unroll
+      for (uint32_t i = 0; i < kPairs; ++i) {
+        const uint32_t p = k * kPairs + i;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(
+            rw, (__attribute__((address_space(3))) void*)&L.wq[i][0][0], 16, w_off,
+            (int)((p < np ? p : np - 1u) * kPairBytes), 0, 0);
+      }
+#pragma unroll
+      for (uint32_t i = 0; i < kPairs / 4u; ++i) {
+        const uint32_t p = k * kPairs + 4u * i + grp;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(
+            rw, (__attribute__((address_space(3))) void*)&L.we[4u * i][0], 4,
+            e_off + (p < np ? p : np - 1u) * kPairBytes, 0, 0, 0);
+      }
+    };
+    for (uint32_t k = 0; k + 1u < kRing; ++k) stage(k);
+    // Before barrier k: chunk k has landed (kRing - 2 later ones may be in flight). After
+    // it every wave is done with chunk k - 1, whose buffer takes chunk k - 1 + kRing.
+    static_assert((kPairs + kPairs / 4u) * (kRing - 2u) == 5u, "the wait below");
+    for (uint32_t k = 0; k < n_bar; ++k) {
+      __builtin_amdgcn_s_waitcnt(0x0f75);  // vmcnt(5)
+      barrier();
+      stage(k + kRing - 1u);
+    }
+    __builtin_amdgcn_s_waitcnt(0x0f70);  // no load into LDS outlives the workgroup
+    return;
+  }
+
+  const uint32_t tt = blockIdx.y * (uint32_t)W + wave;
+  if (tt >= n_tiles) {  // wave-uniform
+    for (uint32_t k = 0; k < n_bar; ++k) barrier();
+    return;
+  }
+
+  // Activation of group g: a unit of each of its two pairs, and the scale of block
+  // 4g + grp; past the row's end (in the last group) the last one's. The lane's part of an
+  // address is a register, the group's a scalar.
+  const __amdgpu_buffer_rsrc_t rq = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)(ws + (uint64_t)tt * np * 1024u), (short)0, 0x7fffffff, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)(ws + act_quant_bytes(n_tiles, nb) + (uint64_t)tt * nb * 64u), (short)0, 0x7fffffff, 0x00020000);
+  const uint32_t in_last = nb - kGroup * (ng - 1u);  // blocks of the last group: 2 or 4
+  const int32_t blocks_left = (int32_t)nb - (int32_t)grp;
+  const uint32_t xq_off = lane * 16u, xs_off = lane * 4u;
+  const uint32_t xs_last = (grp < in_last ? grp : in_last - 1u) * 64u + c * 4u;
+  uint4 xq[4][2];
+  uint32_t xs[4];
+  auto load_x = [&](uint32_t g, int slot) __attribute__((always_inline)) {
+    const uint32_t gl = g < ng ? g : ng - 1u;  // loads past the last group read it again
+    const uint32_t p1 = 2u * gl + 1u < np ? 2u * gl + 1u : np - 1u;
+    xq[slot][0] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rq, xq_off, gl * 2048u, 0));
+    xq[slot][1] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rq, xq_off, p1 * 1024u, 0));
+    xs[slot] = __builtin_amdgcn_raw_buffer_load_b32(rs, gl == ng - 1u ? xs_last : xs_off, gl * 256u, 0);
+  };
+
+  // Weights of a group: 8 quants of row c of each block (unit grp / 2 of the block), the
+  // pairs' dwords 8 and the scale of block grp.
+  const uint32_t f = c / 4u;
+  const uint32_t o_even = c * 64u + ((grp / 2u) ^ f) * 16u + (grp % 2u) * 8u, o_odd = o_even ^ 32u;
+  const uint32_t o_we = (uint32_t)offsetof(RowChunk, we) + c * 4u;
+  const bool s_odd = grp % 2u != 0u;
+  const uint32_t o_s = s_odd ? o_we + (grp / 2u) * 64u + 2u : (grp / 2u) * 1024u + c * 64u + f * 16u;
+  const uint32_t s_step = s_odd ? 128u : 2048u;  // a group on
+  uint2 wb[2][4];
+  uint32_t we[2][2], sw[2];
+  uint32_t a_even = o_even, a_odd = o_odd, a_we = o_we, a_s = o_s;  // in the chunk being read
+  auto at_chunk = [&](uint32_t base) __attribute__((always_inline)) {
+    a_even = base + o_even;
+    a_odd = base + o_odd;
+    a_we = base + o_we;
+    a_s = base + o_s;
+  };
+  auto read_w = [&](int g) __attribute__((always_inline)) {  // group g % kGroups of the chunk
+    const uint8_t* L = (const uint8_t*)ring;
+    const int j = g % kGroups, t = g % 2;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      wb[t][2 * i] = *(const uint2*)(L + a_even + (2 * j + i) * 1024);
+      wb[t][2 * i + 1] = *(const uint2*)(L + a_odd + (2 * j + i) * 1024);
+      we[t][i] = *(const uint32_t*)(L + a_we + (2 * j + i) * 64);
+    }
+    sw[t] = *(const uint16_t*)(L + a_s);
+    a_s += s_step;
+  };
+
+  float acc[4] = {};
+  i32x4 magic = {(int)kMagicBits, (int)kMagicBits, (int)kMagicBits, (int)kMagicBits};
+  __asm__("" : "+v"(magic));
+  const f32x16 zero = {};
+  const uint32_t sel_q = grp == 0u ? 0x05040302u : 0x03020100u;
+  f32x16 P;
+  i32x4 D[4];
+  // Blocks 2h and 2h + 1 of the group in slot: tokens are the MFMA rows.
+  auto dots = [&](int h, int slot) __attribute__((always_inline)) {
+    const uint4 x = xq[slot][h];
+    const uint2* w = wb[slot % 2];
+    const uint32_t w0 = __builtin_amdgcn_perm(we[slot % 2][h], w[2 * h].x, sel_q);
+    auto l64 = [](uint32_t lo, uint32_t hi) { return (long)(((uint64_t)hi << 32) | lo); };
+    D[2 * h] = __builtin_amdgcn_mfma_i32_16x16x32_i8(l64(x.x, x.y), l64(w0, w[2 * h].y), magic, 0, 0, 0);
+    D[2 * h + 1] = __builtin_amdgcn_mfma_i32_16x16x32_i8(
+        l64(x.z, x.w), l64(w[2 * h + 1].x, w[2 * h + 1].y), magic, 0, 0, 0);
+  };
+  auto scales = [&](uint32_t g, int slot) __attribute__((always_inline)) {
+    i32x2 x1 = {(int)xs[slot], 0}, w1 = {(int)sw[slot % 2], 0};
+    if (kTail && (int32_t)(kGroup * g) >= blocks_left) x1[0] = w1[0] = 0;
+    P = __builtin_amdgcn_mfma_f32_16x16x4f16(__builtin_bit_cast(f16x4, x1),
+                                             __builtin_bit_cast(f16x4, w1), zero, 0, 0, 0);
+  };
+  float v[8];
+  auto products = [&](int h) __attribute__((always_inline)) {
+#pragma unroll
+    for (int r = 0; r < 8; ++r) v[r] = __int_as_float(D[2 * h + r / 4][r % 4]) - kMagic;
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int r = 0; r < 8; ++r) v[r] = v[r] * P[8 * h + r];
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto add = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int r = 0; r < 8; ++r) acc[r % 4] = acc[r % 4] + v[r];
+  };
+
+#pragma unroll
+  for (int j = 0; j < 4; ++j) load_x((uint32_t)j, j);
+  barrier();  // chunk 0
+  read_w(0);
+  dots(0, 0);
+  dots(1, 0);
+  scales(0, 0);
+  load_x(4, 0);
+  read_w(1);
+  uint32_t base = 0;
+  auto next_chunk = [&]() __attribute__((always_inline)) {
+    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this wave has read the last one
+    barrier();
+    base = base + sizeof(RowChunk) < sizeof(ring) ? base + (uint32_t)sizeof(RowChunk) : 0u;
+    at_chunk(base);
+  };
+  next_chunk();
+  read_w(2);
+  for (uint32_t k = 0; k < n4; ++k) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      // Group g, while group g + 1's products go through the matrix cores from the operands
+      // in registers, which then take group g + 3's weights and g + 5's activation.
+      const uint32_t g = 4u * k + (uint32_t)j;
+      const int n = (j + 1) % 4;
+      __builtin_amdgcn_sched_barrier(0);
+      products(0);
+      add();
+      __builtin_amdgcn_sched_barrier(0);
+      dots(0, n);
+      __builtin_amdgcn_sched_barrier(0);
+      products(1);
+      scales(g + 1u, n);
+      __builtin_amdgcn_sched_barrier(0);
+      add();
+      __builtin_amdgcn_sched_barrier(0);
+      dots(1, n);
+      load_x(g + 5u, n);
+      if ((j + 3) % kGroups == 0) next_chunk();
+      read_w((j + 3) % 4);
+    }
+  }
+
+  const uint32_t row = row0 + c;
+  if (row >= rows) return;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const uint32_t tok = tt * 16u + 4u * grp + (uint32_t)r;
+    if (tok < n_tokens) M.y[(uint64_t)tok * rows + row] = acc[r];
+  }
+#endif
+}
+
 }  // namespace
 
-// A workgroup takes about as long alone on its CU as with two others (4,096 columns: 25 us
-// at one a CU, 34 us at three), so the kernel wins once every CU has one: at 256
-// workgroups and 4,096 x 4,096 weights 28.1 us against 30.5 for the 16 x 16 kernel (256
+bool gemm_mfma_eligible(const GemvBatch& b, uint32_t cols, uint32_t n_tokens) {
+  if (n_tokens < kGemmMfmaMinTokens || cols % 64u != 0u) return false;
+  for (uint32_t m = 0; m < b.n; ++m)
+    if ((uintptr_t)b.m[m].w % 4u != 0u) return false;
+  return true;
+}
+
+bool gemm_mfma_needs_workspace(const GemvBatch& b, uint32_t cols) {
+  if (cols % 1024u != 0u) return false;
+  for (uint32_t m = 0; m < b.n; ++m)
+    if ((uintptr_t)b.m[m].w % 16u != 0u) return false;
+  return true;
+}
+
+uint64_t gemm_mfma_workspace_bytes(uint32_t cols, uint32_t n_tokens) {
+  const uint32_t n_tiles = (n_tokens + 15u) / 16u, nb = cols / 32u;
+  return act_quant_bytes(n_tiles, nb) + (uint64_t)n_tiles * nb * 16u * 4u;
+}
+
+// A workgroup of the 64 x 64 kernel takes about as long alone on its CU as with two others
+// (4,096 columns: 25 us at one a CU, 34 us at three), so it wins once every CU has one:
+// at 256 workgroups and 4,096 x 4,096 weights 28.1 us against 30.5 for 16 x 16 tiles (256
 // tokens), at 192 27.0 against 24.3 (192 tokens); 2,048 and 14,336 columns turn at the same
-// count (17.4 / 19.4 and 77.5 / 85.7 us at 256). And the tokens have to fill most of its 64:
-// 28,672 rows, 32 tokens 48.5 us against 44.4, 64 tokens 50.7 against 55.5.
+// count (17.4 / 19.4 and 77.5 / 85.7 us at 256). And the tokens have to use more than half
+// of its 64: 28,672 rows, 32 tokens 48.5 us against 47.2, 64 tokens 50 against 69.
 constexpr uint64_t kTileMinWgs = 256;
-constexpr uint32_t kTileMinTokens = 48;
-bool gemm_tile_fills(const GemvBatch& b, uint32_t n_tokens) {
+constexpr uint32_t kTileMinTokens = 33;
+static bool gemm_tile_fills(const GemvBatch& b, uint32_t n_tokens) {
   uint64_t row_tiles = 0;
   for (uint32_t m = 0; m < b.n; ++m) row_tiles += (b.m[m].rows + kTileRows - 1u) / kTileRows;
   const uint64_t wgs = row_tiles * ((n_tokens + 63u) / 64u);
   return n_tokens >= kTileMinTokens && wgs >= kTileMinWgs && wgs < (1ull << 30);
 }
 
-hipError_t launch_gemm_q8_tile(GemvBatch b, uint32_t cols, const float* x, uint32_t n_tokens,
+template <int W>
+static void launch_rows(const GemvBatch& b, uint32_t row_tiles, uint32_t cols, uint32_t n_tokens,
+                 uint32_t n_tiles, const uint8_t* ws, hipStream_t s) {
+  const dim3 grid(row_tiles, (n_tiles + W - 1u) / W);
+  const auto kernel = cols % 512u != 0u ? gemm_q8_rows_kernel<W, true> : gemm_q8_rows_kernel<W, false>;
+  kernel<<<grid, (W + 1) * 64, 0, s>>>(b, cols, n_tokens, n_tiles, ws);
+}
+
+hipError_t launch_gemm_q8_mfma(GemvBatch b, uint32_t cols, const float* x, uint32_t n_tokens,
                                void* workspace, hipStream_t s) {
+  const bool tiles = gemm_tile_fills(b, n_tokens);
+  const uint32_t row_tile = tiles ? kTileRows : kRowTile;
   uint32_t row_tiles = 0;
   for (uint32_t m = 0; m < b.n; ++m) {
     b.m[m].wg0 = row_tiles;
-    row_tiles += (b.m[m].rows + kTileRows - 1u) / kTileRows;
+    row_tiles += (b.m[m].rows + row_tile - 1u) / row_tile;
   }
   for (uint32_t m = b.n; m < (uint32_t)kGemvMaxMats; ++m) b.m[m] = b.m[0];
-  const uint32_t n_tiles = (n_tokens + 15u) / 16u;
+  const uint32_t n_tiles = (n_tokens + 15u) / 16u, token_tiles = (n_tiles + 3u) / 4u;
   const uint64_t items = (uint64_t)n_tiles * 16u * (cols / 8u);
-  q8_act_tile_kernel<<<(uint32_t)((items + kActThreads - 1u) / kActThreads), kActThreads, 0, s>>>(
-      x, cols, n_tokens, n_tiles, (uint8_t*)workspace);
+  const uint32_t act_grid = (uint32_t)((items + kActThreads - 1u) / kActThreads);
+  uint8_t* wsp = (uint8_t*)workspace;
+  if (tiles)
+    q8_act_tile_kernel<false><<<act_grid, kActThreads, 0, s>>>(x, cols, n_tokens, n_tiles, wsp);
+  else
+    q8_act_tile_kernel<true><<<act_grid, kActThreads, 0, s>>>(x, cols, n_tokens, n_tiles, wsp);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  const uint32_t token_tiles = (n_tiles + 3u) / 4u;
-  const uint32_t grid = (row_tiles + 7u) / 8u * 8u * token_tiles;
-  gemm_q8_tile_kernel<<<grid, 256, 0, s>>>(b, cols, n_tokens, n_tiles, row_tiles, token_tiles,
-                                           (const uint8_t*)workspace);
+  if (tiles)
+    gemm_q8_tile_kernel<<<(row_tiles + 7u) / 8u * 8u * token_tiles, 256, 0, s>>>(
+        b, cols, n_tokens, n_tiles, row_tiles, token_tiles, wsp);
+  else if (n_tiles == 1u)
+    launch_rows<1>(b, row_tiles, cols, n_tokens, n_tiles, wsp, s);
+  else if (n_tiles == 2u)
+    launch_rows<2>(b, row_tiles, cols, n_tokens, n_tiles, wsp, s);
+  else
+    launch_rows<4>(b, row_tiles, cols, n_tokens, n_tiles, wsp, s);
   return hipGetLastError();
 }
 

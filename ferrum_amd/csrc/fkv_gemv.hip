@@ -48,7 +48,6 @@ using dev::f16_bits_away;
 using dev::q8_byte;
 
 typedef float f32x4a __attribute__((ext_vector_type(4), aligned(4)));
-typedef int v4i __attribute__((ext_vector_type(4)));
 
 constexpr uint32_t kQ8Bytes = 34;
 constexpr int kGemvWaves = 4;
@@ -354,418 +353,7 @@ hipError_t launch_t(const GemvBatch& b, uint32_t n_wg, uint32_t cols, const floa
   return hipGetLastError();
 }
 
-// ---------------------------------------------------------------------------
-// Batched Q8_0 GEMM on the matrix cores
-// ---------------------------------------------------------------------------
-//
-// For a batch of activation rows (a decode step's sequences, a prefill chunk) the GEMV
-// above takes 4 tokens a launch row, so a 64-token batch reads every weight 16 times.
-// Here the activation is quantized once, into a workspace (q8_act_kernel, the same
-// arithmetic as quantize_x), and gemm_q8_mfma_kernel takes each 32-value block's
-// integer dots of 16 weight rows x 16 tokens from one v_mfma_i32_16x16x32_i8: the int32
-// sums are exact, so they are the reference's sumi whatever the order inside the
-// instruction. Each output then takes acc = acc + f32(sumi) * (w_scale * x_scale) block
-// by block in order from +0, which is dot_q8_row_q8_act (q8_dot.rs:72-109) bit for bit.
-//
-// Workspace, per 16-token tile tt of the batch (tokens past n_tokens quantize to zeros):
-//   quants: 16-byte unit (tt, block pair p, lane) at ((tt * nb/2 + p) * 64 + lane) * 16;
-//           lane = grp*16 + c holds quants grp*8 .. +7 of token tt*16 + c of block 2p
-//           (bytes 0..7) and of block 2p + 1 (bytes 8..15): the MFMA B operand order,
-//           1 KiB per load instruction.
-//   scales: f32 (the binary16 scale's value); token c's scales of blocks 4u .. 4u + 3
-//           in the 16-byte unit (tt * nb/4 + u) * 16 + c after the quants.
-// Needs cols % 1024 == 0 (whole pairs of 16-block chunks) and 16-byte aligned weights.
-
-constexpr uint32_t kMmSub = 16;  // blocks of one set of B operands (a sub-chunk)
-
-// Weight staging of a chunk of CH blocks (CH = 16 or 32): a row's CH * 34 bytes go
-// to LDS at a row stride of CH * 34 + 8 (at CH = 16, 138 dwords: the 16 rows' reads start
-// in 16 distinct even banks). Thread t stages row t / 16: its 16-byte units (t % 16) +
-// 16j and the scales of blocks (t % 16) + 16m.
-template <uint32_t CH>
-struct MmShape {
-  static constexpr uint32_t kRowBytes = CH * kQ8Bytes;
-  static constexpr uint32_t kStride = kRowBytes + 8u;
-  static constexpr uint32_t kRowUnits = kRowBytes / 16u;
-  static constexpr uint32_t kRuns = (kRowUnits + 15u) / 16u;
-  static constexpr uint32_t kScales = CH / 16u;
-};
-
-__host__ __device__ constexpr uint64_t mm_quant_bytes(uint32_t n_tiles, uint32_t nb) {
-  return (uint64_t)n_tiles * nb * 16u * 32u;  // 16 tokens x 32 quants a block
-}
-
-// 64-thread workgroups: measured 1.0-1.4% faster steps than 256 at the same kernel time
-// (Llama-3-8B projections, 64 tokens).
-constexpr uint32_t kActThreads = 64;
-
-__global__ __launch_bounds__(kActThreads) void q8_act_kernel(const float* __restrict__ x,
-                                                             uint32_t cols, uint32_t n_tokens,
-                                                             uint32_t n_tiles,
-                                                             uint8_t* __restrict__ ws) {
-  // Item i: token t = i / (cols/8), values 8j .. 8j + 7 with j = i % (cols/8): piece
-  // grp = j % 4 of block j / 4. The four pieces of a block are a quad of lanes (the
-  // item count per token is a multiple of 4), which exits or stays as a whole.
-  const uint32_t per = cols / 8u, nb = cols / 32u;
-  const uint64_t i = (uint64_t)blockIdx.x * kActThreads + threadIdx.x;
-  if (i >= (uint64_t)n_tiles * 16u * per) return;
-  const uint32_t t = (uint32_t)(i / per), j = (uint32_t)(i % per);
-  f32x4a a = {0.0f, 0.0f, 0.0f, 0.0f}, b = {0.0f, 0.0f, 0.0f, 0.0f};
-  if (t < n_tokens) {
-    const float* src = x + (uint64_t)t * cols + 8u * j;
-    a = *(const f32x4a*)src;
-    b = *(const f32x4a*)(src + 4);
-  }
-  float m = __builtin_fmaxf(__builtin_fabsf(a.x), __builtin_fabsf(a.y));
-  m = __builtin_fmaxf(m, __builtin_fabsf(a.z));
-  m = __builtin_fmaxf(m, __builtin_fabsf(a.w));
-  m = __builtin_fmaxf(m, __builtin_fabsf(b.x));
-  m = __builtin_fmaxf(m, __builtin_fabsf(b.y));
-  m = __builtin_fmaxf(m, __builtin_fabsf(b.z));
-  m = __builtin_fmaxf(m, __builtin_fabsf(b.w));
-  m = __builtin_fmaxf(m, 0.0f);  // all NaN: 0, as the reference's amax = 0 start
-  m = __builtin_fmaxf(m, dev::dpp<0xB1>(m));
-  m = __builtin_fmaxf(m, dev::dpp<0x4E>(m));
-  const float d = div127(m);
-  const float id = (d != 0.0f) ? 1.0f / d : 0.0f;
-  const uint32_t qa = q8_byte(a.x * id) | (q8_byte(a.y * id) << 8) |
-                      (q8_byte(a.z * id) << 16) | (q8_byte(a.w * id) << 24);
-  const uint32_t qb = q8_byte(b.x * id) | (q8_byte(b.y * id) << 8) |
-                      (q8_byte(b.z * id) << 16) | (q8_byte(b.w * id) << 24);
-  const uint32_t tt = t / 16u, c = t % 16u, blk = j / 4u, grp = j % 4u;
-  const uint64_t unit = ((uint64_t)tt * (nb / 2u) + blk / 2u) * 64u + grp * 16u + c;
-  *(uint2*)(ws + unit * 16u + (blk % 2u) * 8u) = make_uint2(qa, qb);
-  if (grp == 0u) {
-    float* xs = (float*)(ws + mm_quant_bytes(n_tiles, nb));
-    xs[(((uint64_t)tt * (nb / 4u) + blk / 4u) * 16u + c) * 4u + blk % 4u] =
-        dev::f16_bits_to_f32(f16_bits_away(d));
-  }
-}
-
-// A workgroup: 16 weight rows of one of the launch's matrices x 4 token tiles (wave w:
-// tile blockIdx.y * 4 + w). The 16 rows' Q8_0 bytes are staged chunk by chunk (CH
-// blocks) into LDS as stored, with their scales as f32 [block][row]; a lane (c, grp)
-// reads its A operand, quants grp*8 .. +7 of row c, from there (one 16-bit realignment
-// for blocks at 2 mod 4). The B operands load one 16-block sub-chunk ahead. The weights:
-// chunk k + 1 loads while chunk k is computed, staged by the four computing waves
-// (without PROD), or by a fifth wave two chunks ahead (PROD: launches that leave one
-// workgroup a CU, where a chunk's weight loads would otherwise hold up the computing
-// waves' B-operand waits). Chunks are 32 blocks wherever the chunk count is even, else 16.
-struct MmB {
-  uint4 q[kMmSub / 2];  // block pairs
-  uint4 s[kMmSub / 4];  // scales of 4 blocks
-};
-
-template <uint32_t CH, bool PF, bool PROD>
-__global__ __launch_bounds__(PROD ? 320 : 256)
-__attribute__((amdgpu_waves_per_eu(CH == 16 ? 4 : 1, 8)))
-void gemm_q8_mfma_kernel(const GemvBatch bat, uint32_t cols, uint32_t n_tokens,
-                         uint32_t n_tiles, const uint8_t* __restrict__ ws) {
-  using S = MmShape<CH>;
-  uint32_t mi = 0;
-#pragma unroll
-  for (int j = 1; j < kGemvMaxMats; ++j)
-    if ((uint32_t)j < bat.n && blockIdx.x >= bat.m[j].wg0) mi = (uint32_t)j;
-  const GemvMat M = mi == 0u ? bat.m[0] : mi == 1u ? bat.m[1] : mi == 2u ? bat.m[2] : bat.m[3];
-  const uint32_t rows = M.rows;
-  const uint32_t row0 = (blockIdx.x - M.wg0) * 16u;
-  const uint32_t nb = cols / 32u;
-  const uint64_t row_bytes = (uint64_t)nb * kQ8Bytes;
-  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-  const uint32_t c = lane & 15u, grp = lane >> 4;
-  const uint32_t tt = blockIdx.y * 4u + wave;
-  const bool on = tt < n_tiles;  // wave-uniform; an idle wave still stages
-  const uint32_t ttc = on ? tt : n_tiles - 1u;
-
-  __shared__ __align__(16) uint8_t s_w[2][16 * S::kStride];
-  __shared__ __align__(16) float s_ws[2][CH][16];
-
-  // Staging (MmShape): a row past the matrix stages its last row (never stored).
-  const uint32_t sr = tid / 16u, sc = tid % 16u;
-  const uint8_t* wsrc = M.w + (uint64_t)(row0 + sr < rows ? row0 + sr : rows - 1u) * row_bytes;
-  uint4 stg[S::kRuns];
-  uint32_t sbits[S::kScales];
-  auto stage_load = [&](uint32_t k) {
-    const uint8_t* p = wsrc + (uint64_t)k * S::kRowBytes;
-#pragma unroll
-    for (uint32_t j = 0; j < S::kRuns; ++j)
-      if (sc + 16u * j < S::kRowUnits) stg[j] = *(const uint4*)(p + (sc + 16u * j) * 16u);
-#pragma unroll
-    for (uint32_t m = 0; m < S::kScales; ++m)
-      sbits[m] = *(const uint16_t*)(p + (sc + 16u * m) * kQ8Bytes);
-  };
-  auto stage_store = [&](uint32_t buf) {
-    uint8_t* d = &s_w[buf][sr * S::kStride + sc * 16u];
-#pragma unroll
-    for (uint32_t j = 0; j < S::kRuns; ++j)
-      if (sc + 16u * j < S::kRowUnits) {
-        uint2* dst = (uint2*)(d + 256u * j);  // 8-byte aligned rows
-        dst[0] = make_uint2(stg[j].x, stg[j].y);
-        dst[1] = make_uint2(stg[j].z, stg[j].w);
-      }
-#pragma unroll
-    for (uint32_t m = 0; m < S::kScales; ++m)
-      s_ws[buf][sc + 16u * m][sr] = dev::f16_bits_to_f32(sbits[m]);
-  };
-  // B operands and x scales of sub-chunk g (blocks 16g .. 16g + 15) for this wave's
-  // token tile.
-  const uint8_t* bq = ws + (((uint64_t)ttc * (nb / 2u)) * 64u + lane) * 16u;
-  const uint8_t* bs = ws + mm_quant_bytes(n_tiles, nb) + (((uint64_t)ttc * (nb / 4u)) * 16u + c) * 16u;
-  auto bq_load = [&](uint32_t g, int p) {
-    return *(const uint4*)(bq + ((uint64_t)g * (kMmSub / 2u) + (uint32_t)p) * 1024u);
-  };
-  auto bs_load = [&](uint32_t g, int u) {
-    return *(const uint4*)(bs + ((uint64_t)g * (kMmSub / 4u) + (uint32_t)u) * 256u);
-  };
-  auto b_load = [&](uint32_t g, MmB& o) {
-#pragma unroll
-    for (int p = 0; p < (int)kMmSub / 2; ++p) o.q[p] = bq_load(g, p);
-#pragma unroll
-    for (int u = 0; u < (int)kMmSub / 4; ++u) o.s[u] = bs_load(g, u);
-  };
-
-  float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-  const uint32_t nsub = nb / kMmSub;
-  // One block's epilogue for this lane's 4 outputs: the reference's
-  // acc + f32(sumi) * (w_scale * x_scale), no fused multiply-add.
-  auto epilogue = [&](const v4i& si, const float4& w4, float xs) {
-    acc[0] = acc[0] + (float)si[0] * (w4.x * xs);
-    acc[1] = acc[1] + (float)si[1] * (w4.y * xs);
-    acc[2] = acc[2] + (float)si[2] * (w4.z * xs);
-    acc[3] = acc[3] + (float)si[3] * (w4.w * xs);
-  };
-  // Chunk k from LDS buffer `buf`, in groups of 4 blocks with B operands o. A group's
-  // four integer dots are issued before its epilogues, which then run in block order.
-  // Each register of o is reloaded with the next sub-chunk's operand
-  // once its last use has issued (one set of registers, a sub-chunk ahead); past the
-  // last sub-chunk the reloads read it again (in bounds, never used), so the loop has no
-  // branch. With PF the next group's A operands and weight scales are read from LDS
-  // before this group's dots, so their latency passes under the epilogues (a lone
-  // wave on its SIMD has nothing else to cover it); without PF each group reads its own
-  // just before use (fewer registers, for launches where several waves share a SIMD).
-  auto compute = [&](uint32_t buf, MmB& o, uint32_t k) {
-    constexpr int kGroups = (int)CH / 4;
-    const uint8_t* wl = &s_w[buf][c * S::kStride + grp * 8u];
-    uint32_t ra[2][4][3];  // a group's A operand dwords as stored (3 at 2 mod 4, else 2)
-    float4 rw[2][4];       // its weight scales of rows grp*4 .. +3
-    auto group_read = [&](int g, int slot) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int b = 4 * g + i;  // the block's parity is its parity in the chunk
-        if (b % 2 == 0) {         // quants at 34b + 2 + 8grp: 2 mod 4
-          const uint32_t* p = (const uint32_t*)(wl + 34 * b);
-          ra[slot][i][0] = p[0];
-          ra[slot][i][1] = p[1];
-          ra[slot][i][2] = p[2];
-        } else {  // 0 mod 4
-          const uint32_t* p = (const uint32_t*)(wl + 34 * b + 2);
-          ra[slot][i][0] = p[0];
-          ra[slot][i][1] = p[1];
-        }
-        if (PF) rw[slot][i] = *(const float4*)&s_ws[buf][b][grp * 4u];
-      }
-    };
-    if (PF) group_read(0, 0);
-#pragma unroll
-    for (int g = 0; g < kGroups; ++g) {
-      const int cur = PF ? (g & 1) : 0;
-      const uint32_t sub = (uint32_t)g / 4u;
-      const int b0 = (4 * g) % (int)kMmSub;  // first block of the group in its sub-chunk
-      const uint32_t gn = k * (CH / kMmSub) + sub + 1u;
-      const uint32_t kn = gn < nsub ? gn : nsub - 1u;
-      if (!PF) group_read(g, cur);
-      long av[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int b = b0 + i;
-        uint32_t lo, hi;
-        if (b % 2 == 0) {
-          lo = __builtin_amdgcn_alignbit(ra[cur][i][1], ra[cur][i][0], 16);
-          hi = __builtin_amdgcn_alignbit(ra[cur][i][2], ra[cur][i][1], 16);
-        } else {
-          lo = ra[cur][i][0];
-          hi = ra[cur][i][1];
-        }
-        av[i] = (long)(((uint64_t)hi << 32) | lo);
-      }
-      // the next group's reads go out before this group's dots and epilogues
-      if (PF && g + 1 < kGroups) group_read(g + 1, cur ^ 1);
-      v4i si[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int b = b0 + i;
-        const uint4 u = o.q[b / 2];
-        const long bv = (b % 2 == 0) ? (long)(((uint64_t)u.y << 32) | u.x)
-                                     : (long)(((uint64_t)u.w << 32) | u.z);
-        const v4i zero = {0, 0, 0, 0};
-        si[i] = __builtin_amdgcn_mfma_i32_16x16x32_i8(av[i], bv, zero, 0, 0, 0);
-      }
-      // the reloads stay after the dots that read the registers they overwrite
-      __builtin_amdgcn_sched_barrier(0);
-      o.q[b0 / 2] = bq_load(kn, b0 / 2);
-      o.q[b0 / 2 + 1] = bq_load(kn, b0 / 2 + 1);
-      const uint4 s4 = o.s[b0 / 4];
-      o.s[b0 / 4] = bs_load(kn, b0 / 4);
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        epilogue(si[i], PF ? rw[cur][i] : *(const float4*)&s_ws[buf][4 * g + i][grp * 4u],
-                 __uint_as_float(i == 0 ? s4.x : i == 1 ? s4.y : i == 2 ? s4.z : s4.w));
-    }
-  };
-
-  const uint32_t nc = nb / CH;  // even (launch_gemm_q8_mfma picks CH so)
-  MmB bo;
-  if (PROD) {
-    // A fifth wave stages the weights: two chunks in flight in its registers, one chunk
-    // into the LDS buffer the four computing waves read next, their scales converted
-    // from there. Its waits on HBM are its own: the computing waves' load counters hold
-    // only their B operands, which a weight load issued before them would otherwise
-    // hold back (loads retire in issue order).
-    // Lane l stages units (l % 4) + 4j of row l / 4; it converts the scales of row l % 16,
-    // blocks l / 16 + 4i.
-    constexpr uint32_t kPer = (S::kRowUnits + 3u) / 4u;
-    constexpr uint32_t kSc = CH / 4u;
-    if (wave == 4u) {
-      const uint32_t pr = lane / 4u, pu = lane % 4u;
-      const uint8_t* psrc =
-          M.w + (uint64_t)(row0 + pr < rows ? row0 + pr : rows - 1u) * row_bytes + pu * 16u;
-      uint4 pst[2][kPer];
-      auto p_load = [&](uint32_t k, int set) {
-        const uint8_t* p = psrc + (uint64_t)k * S::kRowBytes;
-#pragma unroll
-        for (uint32_t j = 0; j < kPer; ++j)
-          if (S::kRowUnits % 4u == 0u || pu + 4u * j < S::kRowUnits)
-            pst[set][j] = *(const uint4*)(p + 64u * j);
-      };
-      auto p_store = [&](int set, uint32_t buf) {
-        uint8_t* d = &s_w[buf][pr * S::kStride + pu * 16u];
-#pragma unroll
-        for (uint32_t j = 0; j < kPer; ++j)
-          if (S::kRowUnits % 4u == 0u || pu + 4u * j < S::kRowUnits) {
-            uint2* dst = (uint2*)(d + 64u * j);  // 8-byte aligned rows
-            dst[0] = make_uint2(pst[set][j].x, pst[set][j].y);
-            dst[1] = make_uint2(pst[set][j].z, pst[set][j].w);
-          }
-        const uint32_t sr = lane % 16u, sb0 = lane / 16u;
-        uint32_t sb[kSc];
-#pragma unroll
-        for (uint32_t i = 0; i < kSc; ++i)
-          sb[i] = *(const uint16_t*)&s_w[buf][sr * S::kStride + (sb0 + 4u * i) * kQ8Bytes];
-#pragma unroll
-        for (uint32_t i = 0; i < kSc; ++i) s_ws[buf][sb0 + 4u * i][sr] = dev::f16_bits_to_f32(sb[i]);
-      };
-      // Loads past the last chunk read the last chunk again (in bounds, never stored),
-      // so every iteration issues set 1's loads before set 0's and the wait before a
-      // set's stores leaves the other set in flight.
-      const uint32_t last = nc - 1u;
-      p_load(0, 0);
-      p_load(1, 1);  // nc >= 2
-      p_store(0, 0);
-      p_load(2u < last ? 2u : last, 0);
-      __syncthreads();  // buffer 0 holds chunk 0
-      for (uint32_t k = 0; k < nc; k += 2) {
-        // set 1 holds chunk k + 1, set 0 chunk k + 2
-        p_store(1, 1);
-        p_load(k + 3u < last ? k + 3u : last, 1);
-        __syncthreads();
-        if (k + 2u < nc) p_store(0, 0);
-        p_load(k + 4u < last ? k + 4u : last, 0);
-        __syncthreads();
-      }
-      return;  // after the last barrier
-    }
-    if (on) b_load(0, bo);
-    __syncthreads();
-    for (uint32_t k = 0; k < nc; k += 2) {
-      if (on) compute(0, bo, k);
-      __syncthreads();
-      if (on) compute(1, bo, k + 1);
-      __syncthreads();
-    }
-  } else {
-  if (on) b_load(0, bo);
-  stage_load(0);
-  stage_store(0);
-  __syncthreads();
-  for (uint32_t k = 0; k < nc; k += 2) {
-    // chunk k (buffer 0) while chunk k + 1's weights load; then chunk k + 1 (buffer 1)
-    stage_load(k + 1);
-    if (on) compute(0, bo, k);
-    stage_store(1);
-    __syncthreads();
-    if (k + 2 < nc) stage_load(k + 2);
-    if (on) compute(1, bo, k + 1);
-    if (k + 2 < nc) stage_store(0);
-    __syncthreads();
-  }
-  }
-
-  if (!on) return;
-  const uint32_t tok = tt * 16u + c;
-  if (tok < n_tokens) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const uint32_t row = row0 + grp * 4u + (uint32_t)r;
-      if (row < rows) M.y[(uint64_t)tok * rows + row] = acc[r];
-    }
-  }
-}
-
 }  // namespace
-
-bool gemm_mfma_eligible(const GemvBatch& b, uint32_t cols, uint32_t n_tokens) {
-  if (n_tokens < kGemmMfmaMinTokens || cols % 1024u != 0u) return false;
-  for (uint32_t m = 0; m < b.n; ++m)
-    if ((uintptr_t)b.m[m].w % 16u != 0u) return false;
-  return true;
-}
-
-uint64_t gemm_mfma_workspace_bytes(uint32_t cols, uint32_t n_tokens) {
-  const uint32_t n_tiles = (n_tokens + 15u) / 16u, nb = cols / 32u;
-  return mm_quant_bytes(n_tiles, nb) + (uint64_t)n_tiles * nb * 16u * 4u;
-}
-
-// Batched launches of at most this many workgroups (one a CU on MI355X's 256 CUs) stage
-// their weights by a fifth wave (gemm_q8_mfma_kernel with PROD).
-#ifndef FKV_GEMM_PRODUCER_WGS
-#define FKV_GEMM_PRODUCER_WGS 256
-#endif
-constexpr uint32_t kGemmProducerWgs = FKV_GEMM_PRODUCER_WGS;
-
-hipError_t launch_gemm_q8_mfma(GemvBatch b, uint32_t cols, const float* x, uint32_t n_tokens,
-                               void* workspace, hipStream_t s) {
-  if (gemm_tile_fills(b, n_tokens)) return launch_gemm_q8_tile(b, cols, x, n_tokens, workspace, s);
-  uint32_t n_wg = 0;
-  for (uint32_t m = 0; m < b.n; ++m) {
-    b.m[m].wg0 = n_wg;
-    n_wg += (b.m[m].rows + 15u) / 16u;
-  }
-  for (uint32_t m = b.n; m < (uint32_t)kGemvMaxMats; ++m) b.m[m] = b.m[0];
-  const uint32_t n_tiles = (n_tokens + 15u) / 16u;
-  const uint64_t items = (uint64_t)n_tiles * 16u * (cols / 8u);
-  q8_act_kernel<<<(uint32_t)((items + kActThreads - 1u) / kActThreads), kActThreads, 0, s>>>(
-      x, cols, n_tokens, n_tiles, (uint8_t*)workspace);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  // 32-block chunks with the A operands and weight scales read a group ahead wherever
-  // the chunk count is even (columns a multiple of 2048), staged by a producer wave
-  // where the launch leaves one workgroup a CU; otherwise 16-block chunks. Measured at
-  // 64 tokens (Llama-3-8B projections, one box, us a call): q/k/v 18.0 (producer 20.7,
-  // 16-block chunks 21.1), attn_output 12.2, gate/up 56.9 (16-block chunks 60.0,
-  // producer 72.1), down 32.0 (no producer 33.6).
-  const uint32_t nb = cols / 32u;
-  const dim3 grid(n_wg, (n_tiles + 3u) / 4u);
-  const bool one_a_cu = (uint64_t)grid.x * grid.y <= kGemmProducerWgs;
-  const uint8_t* wsp = (const uint8_t*)workspace;
-  if (nb % 64u != 0u)
-    gemm_q8_mfma_kernel<16, false, false><<<grid, 256, 0, s>>>(b, cols, n_tokens, n_tiles, wsp);
-  else if (one_a_cu)
-    gemm_q8_mfma_kernel<32, true, true><<<grid, 320, 0, s>>>(b, cols, n_tokens, n_tiles, wsp);
-  else
-    gemm_q8_mfma_kernel<32, true, false><<<grid, 256, 0, s>>>(b, cols, n_tokens, n_tiles, wsp);
-  return hipGetLastError();
-}
 
 size_t gemv_lds_bytes(uint32_t tokens, uint32_t cols) {
   return (size_t)tokens * gemv_padded_blocks(cols / 32u) * kXDw * 4u;

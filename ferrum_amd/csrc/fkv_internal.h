@@ -266,19 +266,17 @@ struct GemvBatch {
 };
 hipError_t launch_gemv_q8(GemvBatch b, uint32_t cols, const float* x, uint32_t n_tokens,
                           hipStream_t s);
-// Batched form on the matrix cores (same results bit for bit): the activation quantized
-// once into a workspace of gemm_mfma_workspace_bytes, then one i8 MFMA per 32-value
-// block of 16 rows x 16 tokens. Eligible for n_tokens >= kGemmMfmaMinTokens, cols a
-// multiple of 1024 and 16-byte aligned weights.
+// Batched form on the matrix cores (fkv_gemm.hip; same results bit for bit): the activation
+// quantized once into a workspace of gemm_mfma_workspace_bytes (16-byte aligned), then i8
+// MFMAs. Eligible for n_tokens >= kGemmMfmaMinTokens, cols a multiple of 64 and 4-byte
+// aligned weights. A call without enough workspace is refused where
+// gemm_mfma_needs_workspace (cols a multiple of 1024, 16-byte aligned weights) and takes
+// the GEMV elsewhere.
 constexpr uint32_t kGemmMfmaMinTokens = 8;
 bool gemm_mfma_eligible(const GemvBatch& b, uint32_t cols, uint32_t n_tokens);
+bool gemm_mfma_needs_workspace(const GemvBatch& b, uint32_t cols);
 uint64_t gemm_mfma_workspace_bytes(uint32_t cols, uint32_t n_tokens);
 hipError_t launch_gemm_q8_mfma(GemvBatch b, uint32_t cols, const float* x, uint32_t n_tokens,
-                               void* workspace, hipStream_t s);
-// The same in 32 x 32 tiles for many tokens (fkv_gemm.hip), with the same workspace, and
-// whether a launch is large enough for it. cols % 64 == 0, weights 4-byte aligned.
-bool gemm_tile_fills(const GemvBatch& b, uint32_t n_tokens);
-hipError_t launch_gemm_q8_tile(GemvBatch b, uint32_t cols, const float* x, uint32_t n_tokens,
                                void* workspace, hipStream_t s);
 
 }  // namespace fkv

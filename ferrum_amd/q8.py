@@ -91,7 +91,7 @@ def gemm_q8_0_batched_workspace_bytes(cols: int, n_tokens: int) -> int:
 def gemm_q8_0_batched(ws, rows, cols: int, x, n_tokens: int, ys, workspace=None,
                       stream=None) -> None:
     """gemm_q8_0_multi on the matrix cores for batches (n_tokens >= 8, cols a multiple of
-    1024, 16-byte aligned weights; otherwise the GEMV), bit-identical. `workspace`: a
+    64, 4-byte aligned weights; otherwise the GEMV), bit-identical. `workspace`: a
     device uint8 tensor of gemm_q8_0_batched_workspace_bytes (allocated here when None)."""
     import torch
     n = len(ws)

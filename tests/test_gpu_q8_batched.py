@@ -129,6 +129,31 @@ def test_large_launches_in_32x32_tiles(rows, cols, n_tokens):
 
 
 @pytest.mark.parametrize("rows,cols,n_tokens,offset", [
+    (17, 64, 8, 0),        # one pair of blocks
+    (33, 192, 16, 4),      # an odd number of pairs, weights 4 mod 16
+    (16, 448, 17, 8),      # a partial last group of blocks
+    (50, 576, 33, 12),     # one pair past 16 blocks
+    (2048, 5632, 11, 0),
+    (16400, 320, 70, 4),   # 32 x 32 tiles, an odd number of pairs
+])
+def test_columns_off_1024_on_the_matrix_cores(rows, cols, n_tokens, offset):
+    """Any multiple of 64 columns and 4-byte aligned weights, non-finite scales among them;
+    the same bits through the GEMV when there is no workspace."""
+    import ferrum_amd as fa
+    rng = np.random.default_rng(rows + cols + n_tokens)
+    w = _weights(rng, rows, cols, special=True)
+    x = (rng.standard_normal((n_tokens, cols)) *
+         rng.choice([1e-4, 1.0, 300.0], (n_tokens, 1))).astype(np.float32)
+    x[1, 40], x[2, cols - 1], x[3, 3] = np.inf, -np.inf, np.nan
+    want = ref.q8_gemm(w, rows, cols, x)
+    assert fa.gemm_q8_0_batched_workspace_bytes(cols, n_tokens) > 0
+    _same(_batched([w], [rows], cols, x, offset=offset)[0], want)
+    import torch
+    small = torch.empty(16, dtype=torch.uint8, device="cuda")
+    _same(_batched([w], [rows], cols, x, offset=offset, workspace=small)[0], want)
+
+
+@pytest.mark.parametrize("rows,cols,n_tokens,offset", [
     (20, 1024, 7, 0),    # too few tokens: GEMV
     (20, 544, 30, 0),    # columns off a multiple of 1024: GEMV
     (20, 1024, 30, 2),   # weights 2 mod 16: GEMV
