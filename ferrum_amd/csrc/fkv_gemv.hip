@@ -363,17 +363,31 @@ size_t gemv_lds_bytes(uint32_t tokens, uint32_t cols) {
 // (under 512 workgroups of 4 waves on 256 CUs) take S = 2, when its LDS fits as well.
 constexpr uint32_t kGemvSplitBelowWgs = 512;
 
-uint32_t gemv_tokens_per_launch(uint32_t n_tokens, uint32_t cols) {
-  uint32_t t = n_tokens >= 3u ? 4u : (n_tokens == 2u ? 2u : 1u);
-  while (t > 1u && gemv_lds_bytes(t, cols) > 65536u) t /= 2u;
-  return t;
+// Tokens a workgroup takes with each weight it reads, for a launch of n_wg workgroups of 16
+// rows. Four read the weights least often, but their ordered sums are four times the VALU
+// work of a wave, so they win only where the launch has workgroups enough at four tokens
+// each; smaller ones run two, twice the workgroups. Llama-3-8B and TinyLlama projections,
+// us at 2 / 4 tokens a workgroup: 384 workgroups (q/k/v) 10.6 / 13.2 for 4 tokens, 22.7 /
+// 23.9 for 12 (1,152 workgroups of 4), 40.3 / 37.9 for 24 (2,304); 256 (attn_output) 8.2 /
+// 10.1, 16.4 / 16.7, 28.3 / 27.2; 704 (TinyLlama gate/up) 10.3 / 10.0, 12.8 / 13.6 for 5
+// (1,408), 22.3 / 20.5 for 12 (2,112); 1,792 (gate/up) 46.9 / 39.7 for 4.
+// Four tokens' activation has to fit 64 KiB of LDS, two tokens' half a CU's 160 (14,336
+// columns, 256 workgroups: 24.0 us for 4 tokens, one a workgroup 38.7, four 29.2).
+constexpr uint64_t kGemvFourMinWgs = 1500;
+constexpr uint32_t kGemvFourMinRowWgs = 512;  // launches of one slice of tokens
+uint32_t gemv_tokens_per_launch(uint32_t n_tokens, uint32_t cols, uint32_t n_wg) {
+  if (n_tokens == 1u) return 1u;
+  const bool four = (uint64_t)n_wg * ((n_tokens + 3u) / 4u) >= kGemvFourMinWgs ||
+                    (n_tokens <= 4u && n_wg >= kGemvFourMinRowWgs);
+  if (n_tokens >= 3u && four && gemv_lds_bytes(4, cols) <= 65536u) return 4u;
+  return gemv_lds_bytes(2, cols) <= kGemvMaxLds / 2u ? 2u : 1u;
 }
 
 hipError_t launch_gemv_q8(GemvBatch b, uint32_t cols, const float* x, uint32_t n_tokens,
                           hipStream_t s) {
   uint32_t n_wg = 0;
   for (uint32_t m = 0; m < b.n; ++m) n_wg += (b.m[m].rows + kRowsPerWg - 1u) / kRowsPerWg;
-  const uint32_t tpl = gemv_tokens_per_launch(n_tokens, cols);
+  const uint32_t tpl = gemv_tokens_per_launch(n_tokens, cols, n_wg);
   const uint32_t S = (tpl == 1u && n_wg < kGemvSplitBelowWgs &&
                       (size_t)gemv_padded_blocks(cols / 32u, 2) * kXDw * 4u <= 65536u)
                          ? 2u

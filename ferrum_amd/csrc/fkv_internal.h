@@ -250,7 +250,6 @@ void* static_scratch(int device);
 // LDS one workgroup may hold on gfx950).
 constexpr size_t kGemvMaxLds = 163840;
 size_t gemv_lds_bytes(uint32_t tokens, uint32_t cols);
-uint32_t gemv_tokens_per_launch(uint32_t n_tokens, uint32_t cols);
 // Up to kGemvMaxMats weight matrices that share the activation x (cols columns): one
 // launch, workgroups [wg0, next wg0) on matrix m; each y[m] as its own launch would give.
 constexpr int kGemvMaxMats = 4;

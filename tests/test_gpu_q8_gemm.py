@@ -96,6 +96,21 @@ def test_matches_oracle(rows, cols, n_tokens):
     _same(_run(w, rows, cols, x), ref.q8_gemm(w, rows, cols, x))
 
 
+@pytest.mark.parametrize("rows,cols,n_tokens", [
+    (8176, 64, 3), (8177, 64, 3),      # 511 and 512 workgroups of 16 rows: 2 and 4 tokens each
+    (11984, 96, 8), (12000, 96, 7),    # 1,498 and 1,500 workgroups of 4 tokens
+    (20, 14336, 3), (20, 16384, 5),    # two tokens' activation past 64 KiB and at 80 KiB of LDS
+    (20, 18432, 3),                    # and past that: one token
+    (8200, 12288, 4),                  # four tokens' past 64 KiB: two
+])
+def test_tokens_a_workgroup(rows, cols, n_tokens):
+    rng = np.random.default_rng(rows + cols + n_tokens)
+    w = _weights(rng, rows, cols)
+    x = (rng.standard_normal((n_tokens, cols)) *
+         rng.choice([1e-4, 1.0, 300.0], (n_tokens, 1))).astype(np.float32)
+    _same(_run(w, rows, cols, x), ref.q8_gemm(w, rows, cols, x))
+
+
 @pytest.mark.parametrize("n_tokens", range(1, 10))
 def test_every_token_count(n_tokens):
     rng = np.random.default_rng(n_tokens)
