@@ -18,6 +18,11 @@ from typing import Optional, Sequence
 
 import numpy as np
 
+try:
+    import torch
+except ImportError:  # the host-only surface works without it
+    torch = None
+
 from . import _lib
 from .errors import check
 
@@ -144,8 +149,12 @@ class PagedConfig:
 
 
 def _stream_ptr(stream) -> int:
+    """The HIP stream handle; None: the current device's current stream. Asked of torch's
+    C layer where CUDA is initialised: torch.cuda.current_stream() builds a Stream object
+    (3.0 us against 0.4), in a call whose launches take 6."""
     if stream is None:
-        import torch
+        if torch.cuda.is_initialized():
+            return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
         return torch.cuda.current_stream().cuda_stream
     if isinstance(stream, int):
         return stream
@@ -153,7 +162,6 @@ def _stream_ptr(stream) -> int:
 
 
 def _dev(t, dtype, name):
-    import torch
     if not isinstance(t, torch.Tensor) or not t.is_cuda:
         raise TypeError(f"{name} must be a device tensor")
     if t.dtype != dtype:
@@ -258,7 +266,6 @@ class PagedKvPool:
 
     # -- device operations --------------------------------------------------
     def append(self, layer: int, k, v, slot_mapping, stream=None) -> None:
-        import torch
         n = slot_mapping.numel()
         row = self.config.n_kv_heads * self.config.head_dim
         if k.numel() != n * row or v.numel() != n * row:
@@ -270,7 +277,6 @@ class PagedKvPool:
 
     def gather_slots(self, layer: int, slot_mapping, out_k, out_v,
                      fmt: int = _lib.GATHER_F32, stream=None) -> None:
-        import torch
         check(self._lib.fkv_gather_slots(self._h, layer,
                                          _dev(slot_mapping, torch.int64, "slot_mapping"),
                                          slot_mapping.numel(), fmt,
@@ -278,7 +284,6 @@ class PagedKvPool:
 
     def gather_tables(self, layer: int, block_tables, ctx_lens, out_offsets, max_ctx_len: int,
                       out_k, out_v, fmt: int = _lib.GATHER_F32, stream=None) -> None:
-        import torch
         n_seqs, max_blocks = block_tables.shape
         check(self._lib.fkv_gather_tables(self._h, layer,
                                           _dev(block_tables, torch.int32, "block_tables"),
@@ -288,7 +293,6 @@ class PagedKvPool:
                                           _stream_ptr(stream)))
 
     def copy_blocks(self, pairs, stream=None) -> None:
-        import torch
         check(self._lib.fkv_copy_blocks(self._h, _dev(pairs, torch.int64, "pairs"),
                                         pairs.shape[0], _stream_ptr(stream)))
 
@@ -317,7 +321,6 @@ class PagedKvPool:
                          scale: Optional[float] = None, workspace=None, stream=None) -> None:
         """q, out: float32 [n_seqs, n_heads, head_dim]; block_tables int32 [n_seqs, max_blocks];
         ctx_lens int32 [n_seqs]."""
-        import torch
         n_seqs, n_heads, d = q.shape
         if d != self.config.head_dim or tuple(out.shape) != tuple(q.shape):
             raise ValueError("q/out must be [n_seqs, n_heads, head_dim]")
@@ -325,11 +328,12 @@ class PagedKvPool:
             raise ValueError("block_tables/ctx_lens must have one row per sequence")
         if scale is None:
             scale = default_scale(d)
-        need = self.attention_workspace_bytes(n_heads, n_seqs, max_ctx_len)
-        ws_ptr, ws_bytes = 0, 0
-        if need:
-            if workspace is None:
+        if workspace is None:
+            need = self.attention_workspace_bytes(n_heads, n_seqs, max_ctx_len)
+            if need:
                 workspace = torch.empty(need, dtype=torch.uint8, device=q.device)
+        ws_ptr, ws_bytes = 0, 0
+        if workspace is not None:  # the library checks its size
             ws_ptr, ws_bytes = workspace.data_ptr(), workspace.numel() * workspace.element_size()
         check(self._lib.fkv_decode_attention(
             self._h, layer, n_heads, _dev(q, torch.float32, "q"), _dev(out, torch.float32, "out"),
@@ -344,7 +348,6 @@ class PagedKvPool:
         """One decode step of one layer (llama.rs:218-247): store k_new/v_new (float32
         [n_seqs, n_kv_heads, head_dim]) at position ctx_lens[s] - 1 through the block
         tables, then decode attention over ctx_lens[s] positions."""
-        import torch
         n_seqs, n_heads, d = q.shape
         if d != self.config.head_dim or tuple(out.shape) != tuple(q.shape):
             raise ValueError("q/out must be [n_seqs, n_heads, head_dim]")
@@ -355,14 +358,14 @@ class PagedKvPool:
             raise ValueError("block_tables/ctx_lens must have one row per sequence")
         if scale is None:
             scale = default_scale(d)
-        n = ctypes.c_uint64()
-        check(self._lib.fkv_append_decode_attention_workspace_size(
-            self._h, n_heads, n_seqs, max_ctx_len, ctypes.byref(n)))
-        need = n.value
+        if workspace is None:
+            n = ctypes.c_uint64()
+            check(self._lib.fkv_append_decode_attention_workspace_size(
+                self._h, n_heads, n_seqs, max_ctx_len, ctypes.byref(n)))
+            if n.value:
+                workspace = torch.empty(n.value, dtype=torch.uint8, device=q.device)
         ws_ptr, ws_bytes = 0, 0
-        if need:
-            if workspace is None:
-                workspace = torch.empty(need, dtype=torch.uint8, device=q.device)
+        if workspace is not None:  # the library checks its size
             ws_ptr, ws_bytes = workspace.data_ptr(), workspace.numel() * workspace.element_size()
         check(self._lib.fkv_append_decode_attention(
             self._h, layer, n_heads, _dev(k_new, torch.float32, "k_new"),
@@ -377,7 +380,6 @@ class PagedKvPool:
         """append_decode_attention with no workspace and no allocation: the split
         partials go to the library's static per-GPU scratch (STATIC_SCRATCH_BYTES).
         Calls that overlap on one GPU race on it; a step needing more is InvalidRequest."""
-        import torch
         n_seqs, n_heads, d = q.shape
         if d != self.config.head_dim or tuple(out.shape) != tuple(q.shape):
             raise ValueError("q/out must be [n_seqs, n_heads, head_dim]")
@@ -403,7 +405,6 @@ class PagedKvPool:
         each sequence's q and k_new are rotated at position ctx_lens[s] - 1 (dims
         (2i, 2i+1) below rope_dim, angle pos / theta^(2i/rope_dim); scalar.rs:167-189)
         before the append and the attention. q is not written back."""
-        import torch
         n_seqs, n_heads, d = q.shape
         if d != self.config.head_dim or tuple(out.shape) != tuple(q.shape):
             raise ValueError("q/out must be [n_seqs, n_heads, head_dim]")
@@ -414,14 +415,14 @@ class PagedKvPool:
             raise ValueError("block_tables/ctx_lens must have one row per sequence")
         if scale is None:
             scale = default_scale(d)
-        n = ctypes.c_uint64()
-        check(self._lib.fkv_rope_append_decode_attention_workspace_size(
-            self._h, n_heads, n_seqs, max_ctx_len, ctypes.byref(n)))
-        need = n.value
+        if workspace is None:
+            n = ctypes.c_uint64()
+            check(self._lib.fkv_rope_append_decode_attention_workspace_size(
+                self._h, n_heads, n_seqs, max_ctx_len, ctypes.byref(n)))
+            if n.value:
+                workspace = torch.empty(n.value, dtype=torch.uint8, device=q.device)
         ws_ptr, ws_bytes = 0, 0
-        if need:
-            if workspace is None:
-                workspace = torch.empty(need, dtype=torch.uint8, device=q.device)
+        if workspace is not None:  # the library checks its size
             ws_ptr, ws_bytes = workspace.data_ptr(), workspace.numel() * workspace.element_size()
         check(self._lib.fkv_rope_append_decode_attention(
             self._h, layer, n_heads, rope_dim, theta, _dev(k_new, torch.float32, "k_new"),
@@ -446,7 +447,6 @@ class PagedKvPool:
         ctx_lens[s] context, each attending causally (crates/model/src/llama.rs:363-378).
         workspace: device scratch for the key-range pieces (allocated here when None);
         split=False passes none, so every workgroup reads its whole key range."""
-        import torch
         rows, n_heads, d = q.shape
         if d != self.config.head_dim or tuple(out.shape) != tuple(q.shape):
             raise ValueError("q/out must be [rows, n_heads, head_dim]")

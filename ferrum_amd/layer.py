@@ -23,7 +23,7 @@ from __future__ import annotations
 
 from typing import Optional
 
-from .kvcache import PagedKvPool, default_scale
+from .kvcache import PagedKvPool, _stream_ptr, default_scale
 from .q8 import gemm_q8_0_batched, gemm_q8_0_batched_workspace_bytes, q8_0_row_bytes
 
 
@@ -66,14 +66,9 @@ class DecodeAttentionLayer:
                     gemm_q8_0_batched_workspace_bytes(self.q_rows, max_seqs))
         self.gws = torch.empty(max(gneed, 16), dtype=torch.uint8, device=dev)
 
-    def _workspace(self, n: int, max_ctx_len: int, stream):
+    def _workspace(self, n: int, max_ctx_len: int, stream, sp: int):
+        """The attention workspace for a call on `stream`, whose handle is sp."""
         import torch
-        if stream is None:
-            ts = torch.cuda.current_stream(self.ws.device)
-        elif isinstance(stream, int):
-            ts = torch.cuda.ExternalStream(stream, device=self.ws.device)
-        else:
-            ts = stream
         need = self.pool.rope_attention_workspace_bytes(self.n_heads, n, max_ctx_len)
         if need > self.ws.numel():
             old = self.ws
@@ -83,7 +78,14 @@ class DecodeAttentionLayer:
             for s in self._ws_streams.values():
                 old.record_stream(s)
             self._ws_streams = {}
-        self._ws_streams[ts.cuda_stream] = ts
+        if sp not in self._ws_streams:
+            if stream is None:
+                ts = torch.cuda.current_stream(self.ws.device)
+            elif isinstance(stream, int):
+                ts = torch.cuda.ExternalStream(stream, device=self.ws.device)
+            else:
+                ts = stream
+            self._ws_streams[sp] = ts
         return self.ws
 
     def forward(self, x, block_tables, ctx_lens, max_ctx_len: int, y, stream=None) -> None:
@@ -95,13 +97,16 @@ class DecodeAttentionLayer:
             raise ValueError("batch or context beyond what the layer was built for")
         if n == 0:
             return
-        q, k, v, attn = self.q[:n], self.k[:n], self.v[:n], self.attn[:n]
+        sp = _stream_ptr(stream)  # once for the three calls
+        q, k, v, attn = self.q, self.k, self.v, self.attn
+        if n < self.max_seqs:
+            q, k, v, attn = q[:n], k[:n], v[:n], attn[:n]
         gemm_q8_0_batched([self.wq, self.wk, self.wv], [self.q_rows, self.kv_rows, self.kv_rows],
-                          self.n_embd, x, n, [q, k, v], workspace=self.gws, stream=stream)
+                          self.n_embd, x, n, [q, k, v], workspace=self.gws, stream=sp)
         self.pool.rope_append_decode_attention(self.layer, k, v, q, attn, block_tables, ctx_lens,
                                                max_ctx_len, self.rope_dim, self.theta,
                                                scale=self.scale,
-                                               workspace=self._workspace(n, max_ctx_len, stream),
-                                               stream=stream)
+                                               workspace=self._workspace(n, max_ctx_len, stream, sp),
+                                               stream=sp)
         gemm_q8_0_batched([self.wo], [self.n_embd], self.q_rows, attn, n, [y],
-                          workspace=self.gws, stream=stream)
+                          workspace=self.gws, stream=sp)

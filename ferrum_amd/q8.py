@@ -17,6 +17,11 @@ from __future__ import annotations
 
 import ctypes
 
+try:
+    import torch
+except ImportError:
+    torch = None
+
 from . import _lib
 from .errors import check
 from .kvcache import _stream_ptr
@@ -34,7 +39,6 @@ def q8_0_row_bytes(cols: int) -> int:
 
 
 def _dev_any(t, dtype, name):
-    import torch
     if not isinstance(t, torch.Tensor) or not t.is_cuda:
         raise TypeError(f"{name} must be a device tensor")
     if t.dtype != dtype:
@@ -46,7 +50,6 @@ def _dev_any(t, dtype, name):
 
 def gemv_q8_0(w, rows: int, cols: int, x, y, stream=None) -> None:
     """Kernels::gemv(DType::Q8_0, w, rows, cols, x, y): y[r] for one activation row."""
-    import torch
     wp, wn = _dev_any(w, torch.uint8, "w")
     xp, xn = _dev_any(x, torch.float32, "x")
     yp, yn = _dev_any(y, torch.float32, "y")
@@ -56,7 +59,6 @@ def gemv_q8_0(w, rows: int, cols: int, x, y, stream=None) -> None:
 def gemm_q8_0(w, rows: int, cols: int, x, n_tokens: int, y, stream=None) -> None:
     """Kernels::gemm(GemmArgs { dtype: Q8_0, w, rows, cols, x, n_tokens, y }):
     y[t * rows + r], each token as gemv_q8_0 of x[t]."""
-    import torch
     wp, wn = _dev_any(w, torch.uint8, "w")
     xp, xn = _dev_any(x, torch.float32, "x")
     yp, yn = _dev_any(y, torch.float32, "y")
@@ -67,7 +69,6 @@ def gemm_q8_0(w, rows: int, cols: int, x, n_tokens: int, y, stream=None) -> None
 def gemm_q8_0_multi(ws, rows, cols: int, x, n_tokens: int, ys, stream=None) -> None:
     """gemm_q8_0 of up to 4 matrices that take the same x (q/k/v, gate/up) in one launch;
     ys[m] equals gemm_q8_0(ws[m], rows[m], cols, x, n_tokens, ys[m]) bit for bit."""
-    import torch
     n = len(ws)
     if len(rows) != n or len(ys) != n:
         raise ValueError("ws, rows and ys must have one entry per matrix")
@@ -93,16 +94,16 @@ def gemm_q8_0_batched(ws, rows, cols: int, x, n_tokens: int, ys, workspace=None,
     """gemm_q8_0_multi on the matrix cores for batches (n_tokens >= 8, cols a multiple of
     64, 4-byte aligned weights; otherwise the GEMV), bit-identical. `workspace`: a
     device uint8 tensor of gemm_q8_0_batched_workspace_bytes (allocated here when None)."""
-    import torch
     n = len(ws)
     if len(rows) != n or len(ys) != n:
         raise ValueError("ws, rows and ys must have one entry per matrix")
     wp = [_dev_any(w, torch.uint8, "w") for w in ws]
     yp = [_dev_any(y, torch.float32, "y") for y in ys]
     xp, xn = _dev_any(x, torch.float32, "x")
-    need = gemm_q8_0_batched_workspace_bytes(cols, n_tokens)
-    if workspace is None and need:
-        workspace = torch.empty(need, dtype=torch.uint8, device=x.device)
+    if workspace is None:
+        need = gemm_q8_0_batched_workspace_bytes(cols, n_tokens)
+        if need:
+            workspace = torch.empty(need, dtype=torch.uint8, device=x.device)
     wsp, wsn = (workspace.data_ptr(), workspace.numel()) if workspace is not None else (0, 0)
     arr_p = ctypes.c_void_p * max(n, 1)
     arr_u = ctypes.c_uint64 * max(n, 1)
