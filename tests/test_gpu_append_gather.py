@@ -109,6 +109,28 @@ def test_append_q8_bit_exact(rounding):
     assert mism.size == 0, f"{mism.size} bytes differ, first at {mism[:4]}"
 
 
+@pytest.mark.parametrize("d,hkv,block_size", [(64, 1, 16), (64, 3, 32), (128, 1, 16), (128, 3, 32)])
+def test_append_q8_windows_bit_exact(d, hkv, block_size):
+    """Windows of 16 tokens whose slots are whole blocks, start off a 4-token group, run
+    backwards, hold gaps and padding, or end early; odd head counts."""
+    from oracle import ref
+    rng = np.random.default_rng(d + hkv)
+    nblk = 256 // block_size
+    slots = np.concatenate([np.arange(16), 32 + np.arange(16)[::-1], 65 + np.arange(20),
+                            128 + 2 * np.arange(9), [-1, 96, 97, -1, 98, 99], 194 + np.arange(3)])
+    slots = slots.astype(np.int64)
+    k = rng.standard_normal((slots.size, hkv, d), dtype=np.float32)
+    v = rng.standard_normal((slots.size, hkv, d), dtype=np.float32)
+    pool, layout = make_pools(1, hkv, d, nblk, block_size=block_size, dtype=8)
+    pool.fill(0x5a)
+    want = np.full(layout.pool_bytes, 0x5a, np.uint8)
+    pool.append(0, to_dev(k), to_dev(v), to_dev(slots))
+    ref.append(layout, want, 0, k, v, slots)
+    mism = np.flatnonzero(pool.read() != want)
+    assert mism.size == 0, f"{mism.size} bytes differ, first at {mism[:4]}"
+    assert pool.take_fault_flags() == 0
+
+
 @pytest.mark.parametrize("dtype,d", [(0, 128), (1, 128), (1, 64), (8, 64), (0, 4), (1, 12)])
 def test_append_gather_roundtrip_scattered(dtype, d):
     """Append through a scattered slot mapping (with -1 padding), gather back by
