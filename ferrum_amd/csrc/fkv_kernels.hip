@@ -635,7 +635,7 @@ __global__ void __launch_bounds__(256) gather_tables_kernel(
 // ---------------------------------------------------------------------------
 
 // Heads per workgroup: F16 one 16-byte unit of each tile a thread (1 at D = 128, 2 at
-// 64); Q8_0 tiles are half the bytes and staged whole, so 4 (8) heads keep as many bytes
+// 64); Q8_0 tiles are half the bytes and taken whole, so 4 (8) heads keep as many bytes
 // in flight per workgroup (one head a workgroup ran at 43% of a device copy).
 constexpr uint32_t gather_heads_per_wg(int dtype, uint32_t d) {
   return dtype == kDtypeF16 ? 256u / (2u * d) : 512u / d;
@@ -655,42 +655,25 @@ struct GatherShape {
 // blocks, 16 x 34 at head_dim 64 and 128 alike.
 constexpr uint32_t kGatherQ8Span = 16u * 34u;
 
-// LDS of the tile path: F16 the V tiles transposed to [token][dim]; Q8_0 both tiles as
-// stored, and for the raw format the workgroup's output records [kv][token][span].
 constexpr int kFmtF32 = 0;  // FKV_GATHER_F32
 constexpr int kFmtRaw = 1;  // FKV_GATHER_RAW
 
-// Q8_0 tiles in LDS: head hl's K tile, then its V tile. For the raw format 16 bytes of
-// padding follow every 256 bytes of a tile and heads start 32 banks apart: the record
-// pass's dword reads of one instruction (lanes of other token groups, blocks and heads,
-// at multiples of 256 bytes in the stored tile) then fall on distinct banks (unpadded:
-// 8 V lanes a bank).
-template <int D, int FMT>
-struct GatherQ8Lds {
-  static constexpr uint32_t kTile = 16u * D + 16u * (D / 32u) * 2u;
-  static constexpr bool kPad = FMT == kFmtRaw;
-  static constexpr uint32_t kTileP = kPad ? kTile + (kTile + 255u) / 256u * 16u : kTile;
-  static constexpr uint32_t kHead = kPad ? (2u * kTileP + 127u) / 256u * 256u + 128u : 2u * kTileP;
-  // byte b of head hl's tile kv
-  __device__ static uint32_t off(uint32_t hl, uint32_t kv, uint32_t b) {
-    return hl * kHead + kv * kTileP + (kPad ? b + (b >> 8) * 16u : b);
-  }
-};
-
+// LDS of the tile path: F16 the V tiles transposed to [token][dim]; Q8_0 to f32 the K and
+// V tile of each head as stored; Q8_0 raw the workgroup's output records
+// [kv][token][span], token rows 560 bytes apart and V's 16 bytes past a whole number of
+// K's (the stores of one instruction then meet few banks twice).
 template <int DT, int D, int FMT>
 struct __align__(16) GatherLds {  // 16-byte unit stores into q
   using S = GatherShape<DT, D>;
-  using Q = GatherQ8Lds<D, FMT>;
+  static constexpr bool kF16 = DT == kDtypeF16;
   static constexpr bool kRec = DT == kDtypeQ8 && FMT == kFmtRaw;
-  union {
-    uint16_t v[S::kHpw][16][S::kVRow];
-    uint8_t q[DT == kDtypeQ8 ? S::kHpw * Q::kHead : 16];
-  };
-  // records: token rows 560 bytes apart, V's 16 bytes past a whole number of K's (the
-  // record pass's stores of one instruction then meet at most 2 to a bank, against 4)
   static constexpr uint32_t kRecRow = kGatherQ8Span + 16u;
   static constexpr uint32_t kRecKv = 16u * kRecRow + 16u;
-  uint8_t rec[kRec ? 2u * kRecKv : 16u];
+  union {
+    uint16_t v[kF16 ? S::kHpw : 1][kF16 ? 16 : 1][S::kVRow];
+    uint8_t q[DT == kDtypeQ8 && !kRec ? S::kHpw * 2 * S::kTile : 16];
+    uint8_t rec[kRec ? 2u * kRecKv : 16u];
+  };
   __device__ uint8_t* rec_at(uint32_t kv, uint32_t o, uint32_t b) {
     return rec + kv * kRecKv + o * kRecRow + b;
   }
@@ -708,6 +691,12 @@ __device__ __forceinline__ void store_f16_unit(uint8_t* dst, uint4 w) {
     ((float4*)dst)[1] = make_float4(f16_bits_to_f32(w.z & 0xffffu), f16_bits_to_f32(w.z >> 16),
                                     f16_bits_to_f32(w.w & 0xffffu), f16_bits_to_f32(w.w >> 16));
   }
+}
+
+// The value of the quad's lane that kCtrl (a quad_perm) names.
+template <int kCtrl>
+__device__ __forceinline__ uint32_t quad_lane(uint32_t x) {
+  return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, kCtrl, 0xf, 0xf, true);
 }
 
 // One tile group: head hl of the workgroup is KV head h (h_ok false past the last head);
@@ -755,144 +744,132 @@ __device__ __forceinline__ void gather_tile(GatherLds<DT, D, FMT>& lds, const Ge
       store_f16_unit<FMT>(out_v + off + (uint64_t)c * kUnitOut, w);
     }
     __syncthreads();  // the LDS is reused by the caller's next tile group
+  } else if constexpr (FMT == kFmtRaw) {
+    // Ferrum's 34-byte blocks (dtype.rs:19-21: f16 scale, then 32 x i8). Bound by HBM, so
+    // what counts is bytes in flight: every thread loads 2 units of K and 2 of V straight
+    // into registers, and LDS holds the output records alone (18 KiB, 8 workgroups a CU;
+    // with the tiles staged too it was 37 KiB and 4). The records then go out as whole
+    // 16-byte units: a token's heads of the workgroup are one contiguous span of its
+    // output row. Blocks start 34 bytes apart, so an even one's quants lie 2 off a dword
+    // bound and an odd one's on it.
+    // Measured with 8 KV heads of 128 dims, 32,192 tokens of 16 sequences (140 MB): 38.8 ->
+    // 30.1 us, 4.65 TB/s.
+    constexpr uint32_t kNb = D / 32u;
+    constexpr uint32_t kQUnits = S::kHpw * D;       // quant units of the heads' K (V) tiles
+    constexpr uint32_t kSUnits = 2u * kNb;          // scale units of a tile
+    static_assert(kQUnits == 512u && S::kHpw * 2u * kSUnits == 64u, "units a thread");
+    uint4 kw[2] = {}, vw[2] = {}, sw = make_uint4(0, 0, 0, 0);
+    const uint32_t s_hl = threadIdx.x / (2u * kSUnits), s_kv = threadIdx.x / kSUnits % 2u,
+                   s_un = threadIdx.x % kSUnits;
+    if (blk_ok) {
+#pragma unroll
+      for (uint32_t i = 0; i < 2; i++) {
+        const uint32_t un = threadIdx.x + 256u * i, h = h0 + un / D, at = un % D * 16u;
+        if (h < g.n_kv_heads) {
+          kw[i] = *(const uint4*)(tile_ptr(g, (uint64_t)blk, layer, 0, h) + at);
+          vw[i] = *(const uint4*)(tile_ptr(g, (uint64_t)blk, layer, 1, h) + at);
+        }
+      }
+      if (threadIdx.x < 64u && h0 + s_hl < g.n_kv_heads)
+        sw = *(const uint4*)(tile_ptr(g, (uint64_t)blk, layer, s_kv, h0 + s_hl) + 16u * D + s_un * 16u);
+    }
+    // 8 scales a unit, in (token, block) order
+    if (threadIdx.x < 64u) {
+      const uint32_t w[4] = {sw.x, sw.y, sw.z, sw.w};
+#pragma unroll
+      for (uint32_t e = 0; e < 8; e++) {
+        const uint32_t at = s_un * 8u + e;
+        *(uint16_t*)lds.rec_at(s_kv, at / kNb, s_hl * (uint32_t)kHeadBytes + at % kNb * 34u) =
+            (uint16_t)(w[e / 2u] >> (16u * (e % 2u)));
+      }
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < 2; i++) {
+      const uint32_t un = threadIdx.x + 256u * i, p = un % D / 64u;
+      const uint32_t head = un / D * (uint32_t)kHeadBytes + 68u * p;  // blocks 2p, 2p + 1
+      {  // K unit (run, token): 8 quants of each block
+        uint8_t* dst = lds.rec_at(0u, un % 16u, head + 2u + un / 16u % 4u * 8u);
+        *(uint16_t*)dst = (uint16_t)kw[i].x;
+        *(uint32_t*)(dst + 2) = (kw[i].x >> 16) | (kw[i].y << 16);
+        *(uint16_t*)(dst + 6) = (uint16_t)(kw[i].y >> 16);
+        ((uint32_t*)(dst + 34))[0] = kw[i].z;
+        ((uint32_t*)(dst + 34))[1] = kw[i].w;
+      }
+      // V unit (token group, dim j): dword mm holds the 4 tokens of dim 16mm + j. A quad of
+      // lanes has 4 dims; lane e takes token e's byte from each (4 x 4 byte transpose).
+      const uint32_t e = threadIdx.x % 4u;
+      uint8_t* dst = lds.rec_at(1u, un / 16u % 4u * 4u + e, head + 2u + un % 16u / 4u * 4u);
+      const uint32_t w[4] = {vw[i].x, vw[i].y, vw[i].z, vw[i].w};
+      const uint32_t sel = 0x0c0c0400u + e * 0x0101u;  // byte e of both operands
+#pragma unroll
+      for (uint32_t mm = 0; mm < 4; mm++) {
+        const uint32_t l0 = quad_lane<0x00>(w[mm]), l1 = quad_lane<0x55>(w[mm]),
+                       l2 = quad_lane<0xAA>(w[mm]), l3 = quad_lane<0xFF>(w[mm]);
+        const uint32_t t = __builtin_amdgcn_perm(l1, l0, sel) |
+                           (__builtin_amdgcn_perm(l3, l2, sel) << 16);
+        uint8_t* to = dst + mm / 2u * 34u + mm % 2u * 16u;
+        if (mm < 2u) {
+          ((uint16_t*)to)[0] = (uint16_t)t;
+          ((uint16_t*)to)[1] = (uint16_t)(t >> 16);
+        } else {
+          *(uint32_t*)to = t;
+        }
+      }
+    }
+    __syncthreads();
+    if (blk_ok) {
+      // The span of the group's heads that exist, at h0 * kHeadBytes = a multiple of 544
+      // bytes into the row: whole 16-byte units where the rows keep that alignment,
+      // dwords otherwise (records are dword multiples).
+      const uint32_t nh = g.n_kv_heads - h0 < (uint32_t)S::kHpw ? g.n_kv_heads - h0 : (uint32_t)S::kHpw;
+      const uint32_t span = nh * (uint32_t)kHeadBytes;
+      const uint64_t col0 = (uint64_t)h0 * kHeadBytes;
+      auto put = [&](auto unit, uint32_t per) {
+        using U = decltype(unit);
+        const uint32_t half = (uint32_t)n * per;
+        for (uint32_t i = threadIdx.x; i < 2u * half; i += 256u) {
+          const uint32_t kv = i >= half ? 1u : 0u, r = i - (kv ? half : 0u);
+          const uint32_t o = r / per, u = r % per;
+          *(U*)((kv ? out_v : out_k) + (row0 + o) * row_bytes + col0 + u * (uint32_t)sizeof(U)) =
+              *(const U*)lds.rec_at(kv, o, u * (uint32_t)sizeof(U));
+        }
+      };
+      if (span == kGatherQ8Span && row_bytes % 16u == 0) put(uint4{}, kGatherQ8Span / 16u);
+      else if (span % 16u == 0 && row_bytes % 16u == 0) put(uint4{}, span / 16u);
+      else put(uint32_t{}, span / 4u);
+    }
+    __syncthreads();
   } else {
-    // Q8_0: both tiles of every head to LDS as stored, then each output unit from there.
+    // Q8_0 to f32: both tiles of every head to LDS as stored, then each output unit from
+    // there.
     for (uint32_t i = threadIdx.x; i < (uint32_t)(S::kHpw * 2 * S::kUnits); i += 256u) {
       const uint32_t hl = i / (2u * S::kUnits), r = i % (2u * S::kUnits);
       const uint32_t kv = r / S::kUnits, un = r % S::kUnits;
       const uint32_t h = h0 + hl;
       if (blk_ok && h < g.n_kv_heads)
-        *(uint4*)&lds.q[GatherQ8Lds<D, FMT>::off(hl, kv, un * 16u)] =
+        *(uint4*)&lds.q[(hl * 2u + kv) * S::kTile + un * 16u] =
             *(const uint4*)(tile_ptr(g, (uint64_t)blk, layer, kv, h) + (uint64_t)un * 16u);
     }
     __syncthreads();
     if (blk_ok) {
-      if constexpr (FMT == kFmtRaw) {
-        // Ferrum's 34-byte blocks (dtype.rs:19-21: f16 scale, then 32 x i8), in two
-        // passes. First each output record is built in LDS: a step is one block b of 4
-        // consecutive tokens 4q .. 4q + 3 of one tile, whose quants come from the staged
-        // tile as whole dwords (K: 8 bytes of a token's run at a time; V: a dword holds
-        // the 4 tokens' bytes of one dim, transposed by byte permutes), written as dwords
-        // plus one 2-byte store (the scale or the last two quants, by b's parity: blocks
-        // start 34 bytes apart, records 4-byte aligned). Then the records go out as
-        // whole 16-byte units: a token's heads of the workgroup are one contiguous span
-        // of its output row (written directly, the 4-byte stores of 64 lanes fell on as
-        // many scattered blocks).
-        // Wave 0 takes the V blocks (64 items: head, token quad, block; a quad's 4 tokens
-        // share each dword read), waves 1-3 the K blocks (256 items: head, token, block),
-        // so no wave runs both paths and all four work (kHpw x kNb = 16 at head_dim 64
-        // and 128 alike).
-        constexpr uint32_t kNb = D / 32u;
-        static_assert(S::kHpw * kNb == 16, "64 V and 256 K items");
-        using Q = GatherQ8Lds<D, FMT>;
-        // byte b of a tile (the padding is inserted between 256-byte spans, and no read
-        // below crosses one)
-        auto tb = [](uint32_t b) { return Q::kPad ? b + (b >> 8) * 16u : b; };
-        // one 34-byte block of token o from its quant dwords qw and its scale
-        auto put = [&](uint32_t kv, uint32_t o, uint32_t hl, uint32_t b, const uint32_t (&qw)[8],
-                       uint32_t sc) {
-          uint8_t* dst = lds.rec_at(kv, o, hl * (uint32_t)kHeadBytes + b * 34u);
-          if (b % 2u) {  // the block starts 2 mod 4: scale, then the quants on dword bounds
-            *(uint16_t*)dst = (uint16_t)sc;
+      // f16_to_f32(scale) * (i8 as f32), scalar.rs:268-275: 8 dims a step
+      constexpr uint32_t kPer = 2u * 16u * (D / 8u);
+      for (uint32_t i = threadIdx.x; i < (uint32_t)S::kHpw * kPer; i += 256u) {
+        const uint32_t hl = i / kPer, r = i % kPer;
+        const uint32_t kv = r / (16u * (D / 8u)), o = (r / (D / 8u)) % 16u, c8 = r % (D / 8u);
+        const uint32_t h = h0 + hl;
+        if (h >= g.n_kv_heads || (int32_t)o >= n) continue;
+        const uint8_t* t = lds.q + (hl * 2u + kv) * S::kTile;
+        const float sc =
+            f16_bits_to_f32(*(const uint16_t*)&t[16u * D + (o * (D / 32u) + c8 / 4u) * 2u]);
+        float x[8];
 #pragma unroll
-            for (uint32_t k = 0; k < 8; k++) *(uint32_t*)(dst + 2 + 4 * k) = qw[k];
-          } else {  // on a dword bound: scale and two quants, then quants two bytes on
-            *(uint32_t*)dst = sc | (qw[0] << 16);
-#pragma unroll
-            for (uint32_t k = 1; k < 8; k++)
-              *(uint32_t*)(dst + 4 * k) = (qw[k - 1] >> 16) | (qw[k] << 16);
-            *(uint16_t*)(dst + 32) = (uint16_t)(qw[7] >> 16);
-          }
-        };
-        if (threadIdx.x < 64u) {
-          const uint32_t hl = threadIdx.x / (4u * kNb), q = (threadIdx.x / kNb) % 4u,
-                         b = threadIdx.x % kNb;
-          if (h0 + hl < g.n_kv_heads && (int32_t)(4u * q) < n) {
-            const uint8_t* t = lds.q + Q::off(hl, 1u, 0u);
-            uint32_t qw[4][8];  // [token][quant dword]
-#pragma unroll
-            for (uint32_t k = 0; k < 8; k++) {  // dims b*32 + 4k .. 4k + 3: m = 2b + k/4
-              const uint32_t m = 2u * b + k / 4u, j0 = (k % 4u) * 4u;
-              uint32_t w[4];
-#pragma unroll
-              for (uint32_t jj = 0; jj < 4; jj++)
-                w[jj] = *(const uint32_t*)&t[tb((m / 4u) * 1024u + (q * 16u + j0 + jj) * 16u + (m % 4u) * 4u)];
-              // 4 x 4 byte transpose: token tt's bytes of dims 4k .. 4k + 3
-              const uint32_t lo01 = __builtin_amdgcn_perm(w[1], w[0], 0x05010400u);
-              const uint32_t hi01 = __builtin_amdgcn_perm(w[1], w[0], 0x07030602u);
-              const uint32_t lo23 = __builtin_amdgcn_perm(w[3], w[2], 0x05010400u);
-              const uint32_t hi23 = __builtin_amdgcn_perm(w[3], w[2], 0x07030602u);
-              qw[0][k] = __builtin_amdgcn_perm(lo23, lo01, 0x05040100u);
-              qw[1][k] = __builtin_amdgcn_perm(lo23, lo01, 0x07060302u);
-              qw[2][k] = __builtin_amdgcn_perm(hi23, hi01, 0x05040100u);
-              qw[3][k] = __builtin_amdgcn_perm(hi23, hi01, 0x07060302u);
-            }
-#pragma unroll
-            for (uint32_t tt = 0; tt < 4; tt++) {
-              const uint32_t o = 4u * q + tt;
-              if ((int32_t)o >= n) break;
-              put(1u, o, hl, b, qw[tt], *(const uint16_t*)&t[tb(16u * D + (o * kNb + b) * 2u)]);
-            }
-          }
-        } else {
-          for (uint32_t i = threadIdx.x - 64u; i < 16u * 16u; i += 192u) {
-            const uint32_t hl = i / (16u * kNb), o = (i / kNb) % 16u, b = i % kNb;
-            if (h0 + hl >= g.n_kv_heads || (int32_t)o >= n) continue;
-            const uint8_t* t = lds.q + Q::off(hl, 0u, 0u);
-            uint32_t qw[8];
-#pragma unroll
-            for (uint32_t gg = 0; gg < 4; gg++) {  // dims b*32 + gg*8 .. +7
-              const uint2 w = *(const uint2*)&t[tb((b / 2u) * 1024u + (gg * 16u + o) * 16u + (b % 2u) * 8u)];
-              qw[2 * gg] = w.x;
-              qw[2 * gg + 1] = w.y;
-            }
-            put(0u, o, hl, b, qw, *(const uint16_t*)&t[tb(16u * D + (o * kNb + b) * 2u)]);
-          }
-        }
-        __syncthreads();
-        // The span of the group's heads that exist, at h0 * kHeadBytes = a multiple of 544
-        // bytes into the row: whole 16-byte units where the rows keep that alignment,
-        // dwords otherwise (records are dword multiples).
-        const uint32_t nh = g.n_kv_heads - h0 < (uint32_t)S::kHpw ? g.n_kv_heads - h0 : (uint32_t)S::kHpw;
-        const uint32_t span = nh * (uint32_t)kHeadBytes;
-        const uint64_t col0 = (uint64_t)h0 * kHeadBytes;
-        if (span % 16u == 0 && row_bytes % 16u == 0) {
-          const uint32_t per = span / 16u;
-          for (uint32_t i = threadIdx.x; i < 2u * (uint32_t)n * per; i += 256u) {
-            const uint32_t kv = i / ((uint32_t)n * per), r = i % ((uint32_t)n * per);
-            const uint32_t o = r / per, u = r % per;
-            *(uint4*)((kv ? out_v : out_k) + (row0 + o) * row_bytes + col0 + u * 16u) =
-                *(const uint4*)lds.rec_at(kv, o, u * 16u);
-          }
-        } else {
-          const uint32_t per = span / 4u;
-          for (uint32_t i = threadIdx.x; i < 2u * (uint32_t)n * per; i += 256u) {
-            const uint32_t kv = i / ((uint32_t)n * per), r = i % ((uint32_t)n * per);
-            const uint32_t o = r / per, u = r % per;
-            *(uint32_t*)((kv ? out_v : out_k) + (row0 + o) * row_bytes + col0 + u * 4u) =
-                *(const uint32_t*)lds.rec_at(kv, o, u * 4u);
-          }
-        }
-      } else {
-        // f16_to_f32(scale) * (i8 as f32), scalar.rs:268-275: 8 dims a step
-        constexpr uint32_t kPer = 2u * 16u * (D / 8u);
-        for (uint32_t i = threadIdx.x; i < (uint32_t)S::kHpw * kPer; i += 256u) {
-          const uint32_t hl = i / kPer, r = i % kPer;
-          const uint32_t kv = r / (16u * (D / 8u)), o = (r / (D / 8u)) % 16u, c8 = r % (D / 8u);
-          const uint32_t h = h0 + hl;
-          if (h >= g.n_kv_heads || (int32_t)o >= n) continue;
-          const uint8_t* t = lds.q + GatherQ8Lds<D, FMT>::off(hl, kv, 0u);  // unpadded
-          const float sc =
-              f16_bits_to_f32(*(const uint16_t*)&t[16u * D + (o * (D / 32u) + c8 / 4u) * 2u]);
-          float x[8];
-#pragma unroll
-          for (uint32_t e = 0; e < 8; e++)
-            x[e] = sc * (float)(int8_t)t[q8_quant_offset(kv, o, c8 * 8u + e, D)];
-          float4* dst = (float4*)((kv ? out_v : out_k) + (row0 + o) * row_bytes +
-                                  (uint64_t)h * kHeadBytes + c8 * 32u);
-          dst[0] = make_float4(x[0], x[1], x[2], x[3]);
-          dst[1] = make_float4(x[4], x[5], x[6], x[7]);
-        }
+        for (uint32_t e = 0; e < 8; e++)
+          x[e] = sc * (float)(int8_t)t[q8_quant_offset(kv, o, c8 * 8u + e, D)];
+        float4* dst = (float4*)((kv ? out_v : out_k) + (row0 + o) * row_bytes +
+                                (uint64_t)h * kHeadBytes + c8 * 32u);
+        dst[0] = make_float4(x[0], x[1], x[2], x[3]);
+        dst[1] = make_float4(x[4], x[5], x[6], x[7]);
       }
     }
     __syncthreads();
