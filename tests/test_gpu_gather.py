@@ -170,3 +170,24 @@ def test_gather_unaligned_outputs(dtype):
     assert np.array_equal(gk[:40].cpu().numpy().view(np.uint8), sk.view(np.uint8))
     assert np.array_equal(gv[:40].cpu().numpy().view(np.uint8), sv.view(np.uint8))
     assert pool.take_fault_flags() == 0
+
+
+@pytest.mark.parametrize("d,hkv", [(128, 2), (128, 5), (128, 6), (64, 4), (64, 10)])
+def test_gather_q8_raw_head_groups_bit_exact(d, hkv):
+    """A last group of heads that is not full: whole units, or dwords where rows are no
+    multiple of 16 bytes; contexts that end inside a block."""
+    from oracle import ref
+    nblk = 40
+    pool, layout, image, rng = _filled_pool(8, d, hkv, nblk, seed=d + hkv)
+    ctx = np.array([33, 5, 256], np.int32)
+    tab = rng.permutation(nblk).astype(np.int32)[:36].reshape(3, 12)
+    tab = np.concatenate([tab, tab[::-1, :4]], axis=1)  # 16 entries a row; blocks may repeat
+    wk, wv, offs = ref.gather_tables(layout, image, 1, tab, ctx, 1)
+    rows = int(ctx.sum())
+    gk, gv = _out(rows, hkv, d, 1, 8, 0), _out(rows, hkv, d, 1, 8, 0)
+    offs = np.asarray(offs, np.int64)[:3]
+    pool.gather_tables(1, to_dev(tab), to_dev(ctx), to_dev(offs), 256, gk, gv, 1)
+    assert pool.take_fault_flags() == 0
+    every = slice(0, rows)
+    assert np.array_equal(_rows(gk.cpu().numpy(), every), _rows(wk, every))
+    assert np.array_equal(_rows(gv.cpu().numpy(), every), _rows(wv, every))
