@@ -24,6 +24,7 @@
 // attn_output 55.1 -> 40.4, gate/up 344 -> 249 (483 TFLOP/s), down 171 -> 125. Three waves
 // a SIMD take 217 cycles a block together; the clock is 1.6-1.8 GHz under that load.
 #include "fkv_device.h"
+#include "fkv_gemm_at.h"
 #include "fkv_q8_act.h"
 
 namespace fkv {
@@ -39,7 +40,7 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x32 __attribute__((ext_vector_type(32)));
 
 constexpr uint32_t kQ8Bytes = 34;
-[[maybe_unused]] constexpr uint32_t kPairBytes = 2 * kQ8Bytes;
+static_assert(gemm_at::kPairBytes == 2 * kQ8Bytes, "a pair of blocks");
 constexpr uint32_t kTileRows = 64;      // weight rows of a workgroup
 [[maybe_unused]] constexpr uint32_t kMagicBits = 0x4b400000u;
 [[maybe_unused]] constexpr float kMagic = 12582912.0f;    // 1.5 * 2^23
@@ -105,7 +106,7 @@ __global__ __launch_bounds__(kActThreads) void q8_act_tile_kernel(const float* _
     ((uint32_t*)(ws + act_quant_bytes(n_tiles, nb)))[at * 16u + c] = dev::f16_bits_away(d);
 }
 
-// A buffer of `bytes` at p; loads past its end give zeros.
+// A buffer of `bytes` at p. Every load stays inside it by its own offsets (gemm_at).
 [[maybe_unused]] __device__ __forceinline__ __amdgpu_buffer_rsrc_t lds_source(const void* p,
                                                                              uint64_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(
@@ -159,12 +160,10 @@ __global__ __launch_bounds__(256, 2) void gemm_q8_tile_kernel(const GemvBatch ba
 
   __shared__ Chunk s0, s1, s2;
 
-  // Staging: loads straight into LDS, 6 a wave and chunk. Rows past the matrix and tokens
-  // past the batch read the last one (never used). Chunks past the row's end read on in
-  // the next row; the resources end where the matrix and the workspace do, and a load past
-  // that gives zeros (its scalar offset counts). So an address is a lane's register and a
-  // scalar that only grows: with every index clamped, down of Llama-3-8B took 129 us
-  // where it takes 122 (512 tokens).
+  // Staging: loads straight into LDS, 6 a wave and chunk. Rows past the matrix, tokens past
+  // the batch and blocks past the row's end read the last one (never used; gemm_at). An
+  // address is a lane's register and a scalar, bounded by one scalar minimum for each of a
+  // chunk's two pairs and one for its activation.
   const uint64_t row_bytes = (uint64_t)nb * kQ8Bytes;
   const uint32_t last_row = rows - 1u - row0;
   const uint32_t t16 = ty * 4u;
@@ -173,30 +172,28 @@ __global__ __launch_bounds__(256, 2) void gemm_q8_tile_kernel(const GemvBatch ba
   const __amdgpu_buffer_rsrc_t rq = lds_source(ws + (uint64_t)t16 * nb * 512u, left * 512u);
   const __amdgpu_buffer_rsrc_t rs =
       lds_source(ws + act_quant_bytes(n_tiles, nb) + (uint64_t)t16 * nb * 64u, left * 64u);
-  auto row_at = [&](uint32_t r) { return (r < last_row ? r : last_row) * (uint32_t)row_bytes; };
-  auto tile_at = [&](uint32_t j) { return t16 + j < n_tiles ? j : n_tiles - 1u - t16; };
+  const uint32_t last_tile = n_tiles - 1u - t16;
   // weights: wave w stages rows 16w .. 16w + 15, 4 lanes a row
-  const uint32_t unit = (lane & 3u) ^ (lane >> 4);
-  const uint32_t w_off = row_at(16u * wave + lane / 4u) + unit * 16u + (unit >= 2u ? 4u : 0u);
+  const uint32_t w_off = gemm_at::tile_weights(wave, lane, last_row, (uint32_t)row_bytes);
   // their dwords 8: waves w and w + 2 pair w (the same ones), a lane a row
-  const uint32_t e_off = row_at(lane) + 32u;
+  const uint32_t e_off = gemm_at::tile_dwords8(lane, last_row, (uint32_t)row_bytes);
   // activation: wave w blocks 2 * (w / 2), + 1 of token half w % 2, and their scales
-  const uint32_t x_tile = tile_at(2u * (wave & 1u) + c32 / 16u) * nb;
-  const uint32_t xq_off = x_tile * 512u + half * 256u + (c32 % 16u) * 16u;
-  const uint32_t xs_off = x_tile * 64u + half * 64u + (c32 % 16u) * 4u;
+  const uint32_t xq_off = gemm_at::tile_quants(wave, lane, last_tile, nb);
+  const uint32_t xs_off = gemm_at::tile_scales(wave, lane, last_tile, nb);
 #define FKV_LDS(p) (__attribute__((address_space(3))) void*)(p)
-  const uint32_t e0 = (wave & 1u) * kPairBytes, xb0 = 2u * (wave >> 1);
+  const uint32_t xb0 = 2u * (wave >> 1);
   auto stage = [&](uint32_t k, Chunk& L) __attribute__((always_inline)) {
-    const uint32_t wo = k * (2u * kPairBytes), b = 4u * k + xb0;
+    const uint32_t wo[2] = {gemm_at::pair(2u * k, np), gemm_at::pair(2u * k + 1u, np)};
+    const uint32_t b = gemm_at::tile_block(k, wave, nb);
 #pragma unroll
     for (uint32_t i = 0; i < 2u; ++i) {
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, FKV_LDS(&L.wq[i][16u * wave][0]), 16, w_off,
-                                               (int)(wo + i * kPairBytes), 0, 0);
+                                               (int)wo[i], 0, 0);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rq, FKV_LDS(&L.xq[wave & 1u][xb0 + i][0][0]), 16,
                                                xq_off, (int)((b + i) * 512u), 0, 0);
     }
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, FKV_LDS(&L.we[wave & 1u][0]), 4, e_off,
-                                             (int)(wo + e0), 0, 0);
+                                             (int)(wave & 1u ? wo[1] : wo[0]), 0, 0);
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, FKV_LDS(&L.xs[wave >> 1][wave & 1u][0][0]), 4,
                                              xs_off, (int)(b * 64u), 0, 0);
   };
@@ -392,26 +389,24 @@ __global__ __launch_bounds__((W + 1) * 64, 4) void gemm_q8_rows_kernel(const Gem
   };
 
   if (wave == (uint32_t)W) {
-    // Rows past the matrix load the last one, chunks past the row's end on in the next row
-    // or, past the matrix, zeros (never used, or met by zero scales).
+    // Rows past the matrix and pairs past the row's end load the last one (never used, or
+    // met by zero scales; gemm_at).
     const uint64_t row_bytes = (uint64_t)nb * kQ8Bytes;
     const uint32_t last_row = rows - 1u - row0;
     const __amdgpu_buffer_rsrc_t rw = lds_source(M.w + row0 * row_bytes, (rows - row0) * row_bytes);
-    auto row_at = [&](uint32_t r) { return (r < last_row ? r : last_row) * (uint32_t)row_bytes; };
-    const uint32_t unit = (lane & 3u) ^ (lane >> 4);
-    const uint32_t w_off = row_at(lane / 4u) + unit * 16u + (unit >= 2u ? 4u : 0u);
-    const uint32_t e_off = row_at(c) + grp * kPairBytes + 32u;
+    const uint32_t w_off = gemm_at::rows_weights(lane, last_row, (uint32_t)row_bytes);
+    const uint32_t e_off = gemm_at::rows_dwords8(lane, last_row, (uint32_t)row_bytes);
     auto stage = [&](uint32_t k) __attribute__((always_inline)) {
       RowChunk& L = ring[k % kRing];
-      const uint32_t o = k * (kPairs * kPairBytes);
 #pragma unroll
       for (uint32_t i = 0; i < kPairs; ++i)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(
             rw, (__attribute__((address_space(3))) void*)&L.wq[i][0][0], 16, w_off,
-            (int)(o + i * kPairBytes), 0, 0);
+            (int)gemm_at::pair(k * kPairs + i, np), 0, 0);
       static_assert(kPairs == 4u, "one load holds the pairs' dwords 8");
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          rw, (__attribute__((address_space(3))) void*)&L.we[0][0], 4, e_off, (int)o, 0, 0);
+          rw, (__attribute__((address_space(3))) void*)&L.we[0][0], 4,
+          e_off + gemm_at::pair(k * kPairs + grp, np), 0, 0, 0);
     };
     for (uint32_t k = 0; k + 1u < kRing; ++k) stage(k);
     // Before barrier k: chunk k has landed (kRing - 2 later ones may be in flight). After
@@ -433,18 +428,19 @@ __global__ __launch_bounds__((W + 1) * 64, 4) void gemm_q8_rows_kernel(const Gem
   }
 
   // Activation of group g: a unit of each of its two pairs, and the scale of block
-  // 4g + grp; zeros past the row's end.
+  // 4g + grp; past the row's end the last one's (never used, or met by zero scales).
   const __amdgpu_buffer_rsrc_t rq = lds_source(ws + (uint64_t)tt * np * 1024u, np * 1024u);
   const __amdgpu_buffer_rsrc_t rs =
       lds_source(ws + act_quant_bytes(n_tiles, nb) + (uint64_t)tt * nb * 64u, nb * 64u);
   const int32_t blocks_left = (int32_t)nb - (int32_t)grp;
-  const uint32_t xq_off = lane * 16u, xs_off = lane * 4u;
+  const uint32_t xq_off = lane * 16u;
   uint4 xq[4][2];
   uint32_t xs[4];
   auto load_x = [&](uint32_t g, int slot) __attribute__((always_inline)) {
-    xq[slot][0] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rq, xq_off, g * 2048u, 0));
-    xq[slot][1] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rq, xq_off, g * 2048u + 1024u, 0));
-    xs[slot] = __builtin_amdgcn_raw_buffer_load_b32(rs, xs_off, g * 256u, 0);
+    xq[slot][0] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rq, xq_off, gemm_at::rows_quants(2u * g, np), 0));
+    xq[slot][1] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rq, xq_off, gemm_at::rows_quants(2u * g + 1u, np), 0));
+    xs[slot] = kTail ? __builtin_amdgcn_raw_buffer_load_b32(rs, gemm_at::rows_scales_lane(g, lane, nb), 0, 0)
+                     : __builtin_amdgcn_raw_buffer_load_b32(rs, lane * 4u, gemm_at::rows_scales(g, nb), 0);
   };
 
   // Weights of a group: 8 quants of row c of each block (unit grp / 2 of the block), the
