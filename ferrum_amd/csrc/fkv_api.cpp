@@ -16,6 +16,7 @@
 #include "../../include/ferrum_kv.h"
 #include "../../include/ferrum_q8.h"
 #include "../../include/ferrum_gguf.h"
+#include "fkv_gemv_plan.h"
 #include "fkv_internal.h"
 
 static_assert(FKV_STATIC_SCRATCH_BYTES == fkv::kStaticScratchBytes,

@@ -38,6 +38,7 @@
 #include <utility>
 
 #include "fkv_device.h"
+#include "fkv_gemv_plan.h"
 #include "fkv_q8_act.h"
 
 namespace fkv {
@@ -53,14 +54,14 @@ constexpr uint32_t kQ8Bytes = 34;
 constexpr int kGemvWaves = 4;
 constexpr int kGemvThreads = 64 * kGemvWaves;
 constexpr int kRowsPerWave = 4;                             // 16 lanes per row
-constexpr uint32_t kRowsPerWg = kGemvWaves * kRowsPerWave;  // 16
-constexpr int kPipe = 4;                                    // 16-block steps in flight
-// LDS dwords per (token, block): aligned q[0..8) | shifted q[0..8) | two tail pairs,
-// aligned (q[8] = 0, xs) and shifted (q[8], xs). Each copy's first 8 dwords are
+constexpr uint32_t kRowsPerWg = kGemvRowsPerWg;
+static_assert(kRowsPerWg == kGemvWaves * kRowsPerWave, "rows of a workgroup");
+constexpr int kPipe = kGemvPipe;
+// A (token, block) record in LDS is kGemvXDw dwords: each copy's first 8 dwords are
 // 16-byte aligned. The tail pairs trade places in blocks with bit 3 set
-// (kTailDw): lanes l and l + 8 read blocks 8 records = 160 dwords apart, a multiple
+// (tail_dw): lanes l and l + 8 read blocks 8 records = 160 dwords apart, a multiple
 // of 32 banks, and would otherwise hit the same banks with their 8-byte tail reads.
-constexpr uint32_t kXDw = 20;
+constexpr uint32_t kXDw = kGemvXDw;
 __device__ __forceinline__ uint32_t tail_dw(bool aligned, uint32_t block) {
   const uint32_t swap = (block >> 3) & 1u;
   return aligned ? 16u + 2u * swap : 18u - 2u * swap;
@@ -70,13 +71,6 @@ __device__ __forceinline__ uint32_t tail_dw(bool aligned, uint32_t block) {
 // passes up front slowed the 3- and 4-token launches).
 constexpr int kXRegs = 2;
 constexpr int kXRegsWide = 8;
-
-// LDS blocks a token: the step count rounded up to whole groups of kPipe iterations
-// (an iteration is S steps of 16 blocks), so every step a group runs reads inside the
-// array.
-__host__ __device__ constexpr uint32_t gemv_padded_blocks(uint32_t nb, uint32_t S = 1) {
-  return (nb + 16u * S * kPipe - 1u) / (16u * S * kPipe) * (16u * S * kPipe);
-}
 
 struct RawBlock {
   uint32_t d[8];
@@ -341,7 +335,7 @@ template <int T, int S, int XR = kXRegs>
 hipError_t launch_t(const GemvBatch& b, uint32_t n_wg, uint32_t cols, const float* x,
                     uint32_t n_tokens, hipStream_t s) {
   const dim3 grid(n_wg, (n_tokens + T - 1u) / T);
-  const size_t lds = (size_t)T * gemv_padded_blocks(cols / 32u, S) * kXDw * 4u;
+  const size_t lds = gemv_lds_bytes(T, cols, S);
   if (lds > 65536u) {
     const hipError_t e = hipFuncSetAttribute((const void*)gemv_q8_kernel<T, S, XR>,
                                              hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -355,50 +349,19 @@ hipError_t launch_t(const GemvBatch& b, uint32_t n_wg, uint32_t cols, const floa
 
 }  // namespace
 
-size_t gemv_lds_bytes(uint32_t tokens, uint32_t cols) {
-  return (size_t)tokens * gemv_padded_blocks(cols / 32u) * kXDw * 4u;
-}
-
-// Launches of one token whose S = 1 grid would leave SIMDs with fewer than two waves
-// (under 512 workgroups of 4 waves on 256 CUs) take S = 2, when its LDS fits as well.
-constexpr uint32_t kGemvSplitBelowWgs = 512;
-
-// Tokens a workgroup takes with each weight it reads, for a launch of n_wg workgroups of 16
-// rows. Four read the weights least often, but their ordered sums are four times the VALU
-// work of a wave, so they win only where the launch has workgroups enough at four tokens
-// each; smaller ones run two, twice the workgroups. Llama-3-8B and TinyLlama projections,
-// us at 2 / 4 tokens a workgroup: 384 workgroups (q/k/v) 10.6 / 13.2 for 4 tokens, 22.7 /
-// 23.9 for 12 (1,152 workgroups of 4), 40.3 / 37.9 for 24 (2,304); 256 (attn_output) 8.2 /
-// 10.1, 16.4 / 16.7, 28.3 / 27.2; 704 (TinyLlama gate/up) 10.3 / 10.0, 12.8 / 13.6 for 5
-// (1,408), 22.3 / 20.5 for 12 (2,112); 1,792 (gate/up) 46.9 / 39.7 for 4.
-// Four tokens' activation has to fit 64 KiB of LDS, two tokens' half a CU's 160 (14,336
-// columns, 256 workgroups: 24.0 us for 4 tokens, one a workgroup 38.7, four 29.2).
-constexpr uint64_t kGemvFourMinWgs = 1500;
-constexpr uint32_t kGemvFourMinRowWgs = 512;  // launches of one slice of tokens
-uint32_t gemv_tokens_per_launch(uint32_t n_tokens, uint32_t cols, uint32_t n_wg) {
-  if (n_tokens == 1u) return 1u;
-  const bool four = (uint64_t)n_wg * ((n_tokens + 3u) / 4u) >= kGemvFourMinWgs ||
-                    (n_tokens <= 4u && n_wg >= kGemvFourMinRowWgs);
-  if (n_tokens >= 3u && four && gemv_lds_bytes(4, cols) <= 65536u) return 4u;
-  return gemv_lds_bytes(2, cols) <= kGemvMaxLds / 2u ? 2u : 1u;
-}
-
 hipError_t launch_gemv_q8(GemvBatch b, uint32_t cols, const float* x, uint32_t n_tokens,
                           hipStream_t s) {
   uint32_t n_wg = 0;
   for (uint32_t m = 0; m < b.n; ++m) n_wg += (b.m[m].rows + kRowsPerWg - 1u) / kRowsPerWg;
-  const uint32_t tpl = gemv_tokens_per_launch(n_tokens, cols, n_wg);
-  const uint32_t S = (tpl == 1u && n_wg < kGemvSplitBelowWgs &&
-                      (size_t)gemv_padded_blocks(cols / 32u, 2) * kXDw * 4u <= 65536u)
-                         ? 2u
-                         : 1u;
+  const GemvCut cut = gemv_cut(n_tokens, cols, n_wg);
+  const uint32_t S = cut.split;
   n_wg = 0;
   for (uint32_t m = 0; m < b.n; ++m) {
     b.m[m].wg0 = n_wg;
     n_wg += (b.m[m].rows + kRowsPerWg / S - 1u) / (kRowsPerWg / S);
   }
   for (uint32_t m = b.n; m < (uint32_t)kGemvMaxMats; ++m) b.m[m] = b.m[0];
-  switch (tpl) {
+  switch (cut.tokens) {
     case 4: return launch_t<4, 1>(b, n_wg, cols, x, n_tokens, s);
     case 2: return launch_t<2, 1, 4>(b, n_wg, cols, x, n_tokens, s);
     default:

@@ -1,0 +1,79 @@
+// How one Q8_0 GEMV launch (fkv_gemv.hip) is cut up: LDS, tokens a workgroup, lanes a row.
+// Plain integer functions of the sizes, for the host and the kernels.
+#pragma once
+#include <cstddef>
+#include <cstdint>
+
+#ifdef __HIPCC__
+#define FKV_PLAN __host__ __device__ constexpr
+#else
+#define FKV_PLAN constexpr
+#endif
+
+namespace fkv {
+
+// LDS one workgroup may hold on gfx950.
+constexpr size_t kGemvMaxLds = 163840;
+constexpr uint32_t kGemvRowsPerWg = 16;  // of a workgroup of 4 waves, 16 lanes a row
+constexpr int kGemvPipe = 4;             // 16-block steps in flight
+// LDS dwords per (token, block): aligned q[0..8) | shifted q[0..8) | two tail pairs,
+// aligned (q[8] = 0, xs) and shifted (q[8], xs).
+constexpr uint32_t kGemvXDw = 20;
+
+// LDS blocks a token: the step count rounded up to whole groups of kGemvPipe iterations
+// (an iteration is S steps of 16 blocks), so every step a group runs reads inside the
+// array.
+FKV_PLAN uint32_t gemv_padded_blocks(uint32_t nb, uint32_t S = 1) {
+  return (nb + 16u * S * kGemvPipe - 1u) / (16u * S * kGemvPipe) * (16u * S * kGemvPipe);
+}
+FKV_PLAN size_t gemv_lds_bytes(uint32_t tokens, uint32_t cols, uint32_t S = 1) {
+  return (size_t)tokens * gemv_padded_blocks(cols / 32u, S) * kGemvXDw * 4u;
+}
+
+// tokens: those a workgroup takes with each weight it reads; split: 2 where the 16-lane
+// rows of a wave take every other step of half the rows, twice the workgroups.
+struct GemvCut {
+  uint32_t tokens, split;
+};
+
+// Launches of one token whose S = 1 grid would leave SIMDs with fewer than two waves
+// (under 512 workgroups of 4 waves on 256 CUs) take S = 2, when its LDS fits as well.
+constexpr uint32_t kGemvSplitBelowWgs = 512;
+FKV_PLAN uint32_t gemv_split(uint32_t cols, uint32_t n_wg) {
+  return n_wg < kGemvSplitBelowWgs && gemv_lds_bytes(1, cols, 2) <= 65536u ? 2u : 1u;
+}
+
+// Tokens a workgroup takes with each weight it reads, for a launch of n_wg workgroups of 16
+// rows. Four read the weights least often, but their ordered sums are four times the VALU
+// work of a wave, so they win only where the launch has workgroups enough at four tokens
+// each; smaller ones run two, twice the workgroups. Llama-3-8B and TinyLlama projections,
+// us at 2 / 4 tokens a workgroup: 384 workgroups (q/k/v) 10.6 / 13.2 for 4 tokens, 22.7 /
+// 23.9 for 12 (1,152 workgroups of 4), 40.3 / 37.9 for 24 (2,304); 256 (attn_output) 8.2 /
+// 10.1, 16.4 / 16.7, 28.3 / 27.2; 704 (TinyLlama gate/up) 10.3 / 10.0, 12.8 / 13.6 for 5
+// (1,408), 22.3 / 20.5 for 12 (2,112); 1,792 (gate/up) 46.9 / 39.7 for 4.
+// Four tokens' activation has to fit 64 KiB of LDS, two tokens' half a CU's 160.
+constexpr uint64_t kGemvFourMinWgs = 1500;
+constexpr uint32_t kGemvFourMinRowWgs = 512;  // launches of one slice of tokens
+// Where two tokens' activation takes more than 64 KiB (12,320 to 16,384 columns) a CU holds
+// two workgroups of two tokens, and a launch that leaves most of them out is bound by the
+// chain of a row's ordered sum: one token with split rows has half of it. 14,336 columns, us
+// at one / two tokens: 16 workgroups of rows and 8 tokens 9.5 / 13.9, 32 and 8 (256) 12.0 /
+// 14.2, 64 and 6 (384) 14.6 / 14.4, 64 and 8 (512) 17.0 / 14.4, 256 and 4 (1,024) 40.7 / 25.9.
+constexpr uint64_t kGemvOneMaxWgs = 384;
+FKV_PLAN uint32_t gemv_tokens(uint32_t n_tokens, uint32_t cols, uint32_t n_wg) {
+  if (n_tokens == 1u) return 1u;
+  const bool four = (uint64_t)n_wg * ((n_tokens + 3u) / 4u) >= kGemvFourMinWgs ||
+                    (n_tokens <= 4u && n_wg >= kGemvFourMinRowWgs);
+  if (n_tokens >= 3u && four && gemv_lds_bytes(4, cols) <= 65536u) return 4u;
+  if (gemv_lds_bytes(2, cols) <= 65536u) return 2u;
+  return gemv_lds_bytes(2, cols) <= kGemvMaxLds / 2u && (uint64_t)n_wg * n_tokens > kGemvOneMaxWgs
+             ? 2u
+             : 1u;
+}
+
+FKV_PLAN GemvCut gemv_cut(uint32_t n_tokens, uint32_t cols, uint32_t n_wg) {
+  const uint32_t t = gemv_tokens(n_tokens, cols, n_wg);
+  return GemvCut{t, t == 1u ? gemv_split(cols, n_wg) : 1u};
+}
+
+}  // namespace fkv

@@ -246,10 +246,8 @@ void* static_scratch(int device);
 
 // Q8_0 weight GEMV/GEMM (fkv_gemv.hip): y[t][r] = dot_q8_row_q8_act(w row r, x[t]
 // quantized) for t < n_tokens, r < rows; w rows of cols/32 34-byte blocks (w even,
-// x 4-byte aligned, cols % 32 == 0, gemv_lds_bytes(1, cols) <= kGemvMaxLds: the
-// LDS one workgroup may hold on gfx950).
-constexpr size_t kGemvMaxLds = 163840;
-size_t gemv_lds_bytes(uint32_t tokens, uint32_t cols);
+// x 4-byte aligned, cols % 32 == 0, gemv_lds_bytes(1, cols) <= kGemvMaxLds;
+// fkv_gemv_plan.h).
 // Up to kGemvMaxMats weight matrices that share the activation x (cols columns): one
 // launch, workgroups [wg0, next wg0) on matrix m; each y[m] as its own launch would give.
 constexpr int kGemvMaxMats = 4;

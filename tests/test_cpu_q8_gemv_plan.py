@@ -1,0 +1,38 @@
+"""CPU: how a Q8_0 GEMV launch is cut up (ferrum_amd/csrc/fkv_gemv_plan.h) at sizes whose
+better cut was measured; the cut changes no result, so only its choice is checked."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+pytestmark = pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
+
+
+def _cuts(tmp_path, sizes):
+    exe = tmp_path / "gemv_plan_print"
+    subprocess.run(["g++", "-O2", "-std=c++17", "-Wall", "-o", str(exe),
+                    os.path.join(HERE, "gemm", "gemv_plan_print.cpp")], check=True)
+    text = "".join("%d %d %d\n" % s for s in sizes)
+    out = subprocess.run([str(exe)], input=text, capture_output=True, text=True, check=True)
+    return [tuple(map(int, line.split())) for line in out.stdout.splitlines()]
+
+
+def test_wide_matrices_of_few_rows_take_one_token(tmp_path):
+    """(rows, cols, tokens) -> (tokens a workgroup, row split). us at one / two tokens."""
+    want = {
+        (16, 14336, 2): (1, 2),       # 8.6 / 13.1
+        (16, 14336, 128): (1, 2),     # 9.5 / 14.0
+        (256, 12352, 8): (1, 2),      # 9.4 / 13.8
+        (1024, 16384, 3): (1, 2),     # 12.2 / 15.6
+        (2048, 14336, 2): (1, 2),     # 12.8 / 14.8
+        (4096, 14336, 2): (2, 1),     # 24.6 / 19.9
+        (1024, 14336, 8): (2, 1),     # 17.0 / 14.4
+        (256, 14336, 64): (2, 1),     # 28.8 / 19.0
+        (16, 12288, 8): (2, 1),       # two tokens within 64 KiB
+        (16, 16416, 8): (1, 2),       # two tokens past half a CU's LDS
+        (16, 14336, 1): (1, 2),
+    }
+    got = _cuts(tmp_path, list(want))
+    assert dict(zip(want, got)) == want

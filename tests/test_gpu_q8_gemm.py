@@ -99,8 +99,9 @@ def test_matches_oracle(rows, cols, n_tokens):
 @pytest.mark.parametrize("rows,cols,n_tokens", [
     (8176, 64, 3), (8177, 64, 3),      # 511 and 512 workgroups of 16 rows: 2 and 4 tokens each
     (11984, 96, 8), (12000, 96, 7),    # 1,498 and 1,500 workgroups of 4 tokens
-    (20, 14336, 3), (20, 16384, 5),    # two tokens' activation past 64 KiB and at 80 KiB of LDS
-    (20, 18432, 3),                    # and past that: one token
+    (20, 14336, 3), (20, 16384, 5),    # two tokens' activation past 64 KiB: one, few workgroups,
+    (2048, 14336, 3), (2050, 16384, 3),  # up to 384 workgroups of one; past that two (80 KiB)
+    (20, 18432, 3),                    # past 80 KiB: one token
     (8200, 12288, 4),                  # four tokens' past 64 KiB: two
 ])
 def test_tokens_a_workgroup(rows, cols, n_tokens):
