@@ -46,14 +46,31 @@ FKV_PLAN uint32_t gemv_split(uint32_t cols, uint32_t n_wg) {
 // Tokens a workgroup takes with each weight it reads, for a launch of n_wg workgroups of 16
 // rows. Four read the weights least often, but their ordered sums are four times the VALU
 // work of a wave, so they win only where the launch has workgroups enough at four tokens
-// each; smaller ones run two, twice the workgroups. Llama-3-8B and TinyLlama projections,
-// us at 2 / 4 tokens a workgroup: 384 workgroups (q/k/v) 10.6 / 13.2 for 4 tokens, 22.7 /
-// 23.9 for 12 (1,152 workgroups of 4), 40.3 / 37.9 for 24 (2,304); 256 (attn_output) 8.2 /
-// 10.1, 16.4 / 16.7, 28.3 / 27.2; 704 (TinyLlama gate/up) 10.3 / 10.0, 12.8 / 13.6 for 5
-// (1,408), 22.3 / 20.5 for 12 (2,112); 1,792 (gate/up) 46.9 / 39.7 for 4.
+// each; smaller ones run two, twice the workgroups. us at 2 / 4 tokens a workgroup (w:
+// workgroups of four):
+// - up to 4 tokens, 4,096 columns: 6,144 rows 10.7 / 12.9 (384), 8,192 13.4 / 13.2 (512),
+//   11,264 19.3 / 17.4 (704), 28,672 45.1 / 36.1;
+// - over 4,096 columns a CU holds two workgroups of four, and two tokens win up to about
+//   1,500 of them: 5,632 columns, 8,192 rows 31.2 / 32.3 for 8 tokens (w 1,024), 44.1 /
+//   45.7 (11,264 rows, 1,408), 64.2 / 60.9 (16,384 rows, 2,048);
+// - narrower ones turn from about 700 workgroups of four, and there by whole rounds of the
+//   256 CUs, a round of four costing 1.8 of two: 2,048 columns 9.3 / 9.0 (4,096 rows, 12
+//   tokens, w 768), 12.9 / 11.8 (20 tokens, 1,280), but 9.5 / 10.2 (8,192 rows, 5 tokens: 4
+//   rounds against 6); 4,096 columns 20.1 / 18.1 (8,192 rows, 7 tokens, 1,024), 20.8 / 21.8
+//   (6,144 rows, 12 tokens: 5 against 9), 30.4 / 25.5 (11,264 rows, 7 tokens: 6 against 11).
 // Four tokens' activation has to fit 64 KiB of LDS, two tokens' half a CU's 160.
 constexpr uint64_t kGemvFourMinWgs = 1500;
+constexpr uint64_t kGemvFourMinWgsNarrow = 700;
 constexpr uint32_t kGemvFourMinRowWgs = 512;  // launches of one slice of tokens
+FKV_PLAN bool gemv_four_wins(uint32_t n_tokens, uint32_t cols, uint32_t n_wg) {
+  if (n_tokens <= 4u) return n_tokens >= 3u && n_wg >= kGemvFourMinRowWgs;
+  const uint64_t four = (uint64_t)n_wg * ((n_tokens + 3u) / 4u),
+                 two = (uint64_t)n_wg * ((n_tokens + 1u) / 2u);
+  if (four >= kGemvFourMinWgs) return true;
+  const bool narrow = 3u * gemv_lds_bytes(4, cols) <= kGemvMaxLds;
+  return narrow && four >= kGemvFourMinWgsNarrow &&
+         9u * ((four + 255u) / 256u) < 5u * ((two + 255u) / 256u);
+}
 // Where two tokens' activation takes more than 64 KiB (12,320 to 16,384 columns) a CU holds
 // two workgroups of two tokens, and a launch that leaves most of them out is bound by the
 // chain of a row's ordered sum: one token with split rows has half of it. 14,336 columns, us
@@ -62,9 +79,7 @@ constexpr uint32_t kGemvFourMinRowWgs = 512;  // launches of one slice of tokens
 constexpr uint64_t kGemvOneMaxWgs = 384;
 FKV_PLAN uint32_t gemv_tokens(uint32_t n_tokens, uint32_t cols, uint32_t n_wg) {
   if (n_tokens == 1u) return 1u;
-  const bool four = (uint64_t)n_wg * ((n_tokens + 3u) / 4u) >= kGemvFourMinWgs ||
-                    (n_tokens <= 4u && n_wg >= kGemvFourMinRowWgs);
-  if (n_tokens >= 3u && four && gemv_lds_bytes(4, cols) <= 65536u) return 4u;
+  if (gemv_lds_bytes(4, cols) <= 65536u && gemv_four_wins(n_tokens, cols, n_wg)) return 4u;
   if (gemv_lds_bytes(2, cols) <= 65536u) return 2u;
   return gemv_lds_bytes(2, cols) <= kGemvMaxLds / 2u && (uint64_t)n_wg * n_tokens > kGemvOneMaxWgs
              ? 2u

@@ -36,3 +36,29 @@ def test_wide_matrices_of_few_rows_take_one_token(tmp_path):
     }
     got = _cuts(tmp_path, list(want))
     assert dict(zip(want, got)) == want
+
+
+def test_two_or_four_tokens(tmp_path):
+    """(rows, cols, tokens) -> tokens a workgroup. us at two / four tokens."""
+    want = {
+        (11264, 4096, 7): 4,     # 30.4 / 25.5
+        (11264, 4096, 8): 4,     # 30.9 / 26.4
+        (8192, 4096, 7): 4,      # 20.1 / 18.1
+        (4096, 2048, 20): 4,     # 12.9 / 11.8
+        (1024, 832, 64): 4,      # 10.0 / 9.4
+        (256, 1536, 256): 4,     # 10.2 / 9.6
+        (6144, 3072, 10): 2,     # 17.7 / 19.4
+        (3072, 2752, 24): 2,     # 19.0 / 20.3
+        (11264, 2048, 5): 2,     # 11.9 / 12.7
+        (2048, 2048, 8): 2,      # latency of few workgroups
+        (8192, 5632, 8): 2,      # 31.2 / 32.3
+        (11264, 5632, 6): 2,     # 35.5 / 40.2
+        (16384, 5632, 8): 4,     # 64.2 / 60.9
+        (8192, 4096, 3): 4,      # 12.3 / 12.1
+        (6144, 4096, 4): 2,      # 10.7 / 12.9
+        (28672, 4096, 2): 2,
+        (28672, 8192, 8): 2,     # four past 64 KiB of LDS
+    }
+    got = _cuts(tmp_path, list(want))
+    assert {k: c[0] for k, c in zip(want, got)} == want
+    assert all(c[1] == 1 for c in got)
