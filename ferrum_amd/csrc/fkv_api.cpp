@@ -1517,7 +1517,8 @@ int32_t fkv_gemm_q8_0_batched(uint32_t n_mats, const void* const* w, const uint6
   if (eligible && (small || !aligned) && fkv::gemm_mfma_needs_workspace(b, (uint32_t)cols))
     return fail(FKV_ERR_INVALID,
                 small ? "gemm workspace too small" : "gemm workspace must be 16-byte aligned");
-  if (!eligible || small || !aligned) {
+  if (!eligible || small || !aligned ||
+      !fkv::gemm_mfma_pays(b, (uint32_t)cols, (uint32_t)n_tokens)) {
     FKV_HIP(fkv::launch_gemv_q8(b, (uint32_t)cols, x, (uint32_t)n_tokens, (hipStream_t)stream),
             "gemv launch");
     return ok();

@@ -25,6 +25,7 @@
 // a SIMD take 217 cycles a block together; the clock is 1.6-1.8 GHz under that load.
 #include "fkv_device.h"
 #include "fkv_gemm_at.h"
+#include "fkv_gemv_plan.h"
 #include "fkv_q8_act.h"
 
 namespace fkv {
@@ -577,6 +578,12 @@ bool gemm_mfma_needs_workspace(const GemvBatch& b, uint32_t cols) {
   for (uint32_t m = 0; m < b.n; ++m)
     if ((uintptr_t)b.m[m].w % 16u != 0u) return false;
   return true;
+}
+
+bool gemm_mfma_pays(const GemvBatch& b, uint32_t cols, uint32_t n_tokens) {
+  uint32_t n_wg = 0;
+  for (uint32_t m = 0; m < b.n; ++m) n_wg += (b.m[m].rows + kGemvRowsPerWg - 1u) / kGemvRowsPerWg;
+  return !gemv_runs_at_once(n_tokens, cols, n_wg);
 }
 
 uint64_t gemm_mfma_workspace_bytes(uint32_t cols, uint32_t n_tokens) {

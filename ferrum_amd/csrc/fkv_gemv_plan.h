@@ -91,4 +91,20 @@ FKV_PLAN GemvCut gemv_cut(uint32_t n_tokens, uint32_t cols, uint32_t n_wg) {
   return GemvCut{t, t == 1u ? gemv_split(cols, n_wg) : 1u};
 }
 
+// Batches (8 tokens or more) that the matrix cores could take as well (fkv_gemm.hip): a GEMV
+// all of whose workgroups run at once, up to three a CU, is the quicker one. It is one
+// launch where those are two, and its chain of ordered sums is half as long a block. us as
+// a GEMV / on the matrix cores, w its workgroups: 256 rows of 576 columns 3.7 / 5.8 (8
+// tokens, w 64), 6.2 / 6.6 (128, 1,024), 10.4 / 6.8 (256, 2,048); 1,024 of 4,096 9.3 / 10.7
+// (24, 768), 11.2 / 10.4 (32, 1,024); 2,048 of 2,752 8.6 / 8.7 (12, 768), 10.3 / 8.6 (16,
+// 1,024); 256 of 14,336 8.9 / 22.4 (8, 128).
+constexpr uint64_t kGemvAtOnceWgsPerCu = 3;
+FKV_PLAN bool gemv_runs_at_once(uint32_t n_tokens, uint32_t cols, uint32_t n_wg) {
+  const GemvCut c = gemv_cut(n_tokens, cols, n_wg);
+  if (c.tokens == 4u) return false;  // over 1,300 workgroups of two
+  const uint64_t wgs = (uint64_t)n_wg * c.split * ((n_tokens + c.tokens - 1u) / c.tokens);
+  const uint64_t held = kGemvMaxLds / gemv_lds_bytes(c.tokens, cols, c.split);
+  return wgs <= 256u * (held < kGemvAtOnceWgsPerCu ? held : kGemvAtOnceWgsPerCu);
+}
+
 }  // namespace fkv

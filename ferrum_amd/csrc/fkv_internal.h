@@ -266,12 +266,13 @@ hipError_t launch_gemv_q8(GemvBatch b, uint32_t cols, const float* x, uint32_t n
 // Batched form on the matrix cores (fkv_gemm.hip; same results bit for bit): the activation
 // quantized once into a workspace of gemm_mfma_workspace_bytes (16-byte aligned), then i8
 // MFMAs. Eligible for n_tokens >= kGemmMfmaMinTokens, cols a multiple of 64 and 4-byte
-// aligned weights. A call without enough workspace is refused where
-// gemm_mfma_needs_workspace (cols a multiple of 1024, 16-byte aligned weights) and takes
-// the GEMV elsewhere.
+// aligned weights; launches that the GEMV is quicker for (gemm_mfma_pays) run that. A call
+// without enough workspace is refused where gemm_mfma_needs_workspace (cols a multiple of
+// 1024, 16-byte aligned weights) and takes the GEMV elsewhere.
 constexpr uint32_t kGemmMfmaMinTokens = 8;
 bool gemm_mfma_eligible(const GemvBatch& b, uint32_t cols, uint32_t n_tokens);
 bool gemm_mfma_needs_workspace(const GemvBatch& b, uint32_t cols);
+bool gemm_mfma_pays(const GemvBatch& b, uint32_t cols, uint32_t n_tokens);
 uint64_t gemm_mfma_workspace_bytes(uint32_t cols, uint32_t n_tokens);
 hipError_t launch_gemm_q8_mfma(GemvBatch b, uint32_t cols, const float* x, uint32_t n_tokens,
                                void* workspace, hipStream_t s);

@@ -80,9 +80,10 @@ int32_t fkv_gemm_q8_0_multi(uint32_t n_mats, const void* const* w, const uint64_
  * `workspace`, and i8 MFMAs give a 32-value block's exact integer dots for 16 x 16 or
  * 32 x 32 outputs; each output then accumulates f32(sumi) * (w_scale * x_scale) block by
  * block in order, as dot_q8_row_q8_act does.
- * That path runs when n_tokens >= 8, cols is a multiple of 64 and every w is 4-byte
- * aligned; other calls run the GEMV kernel (workspace unused). Same checks, strings
- * and order as fkv_gemm_q8_0_multi; then, for a call that takes the matrix-core path, the
+ * That path takes calls with n_tokens >= 8, cols a multiple of 64 and every w 4-byte
+ * aligned, unless the GEMV runs all of its workgroups at once and is the quicker one;
+ * other calls run the GEMV kernel (workspace unused). Same checks, strings and order as
+ * fkv_gemm_q8_0_multi; then, for n_tokens, cols and w of the matrix-core path, the
  * workspace must hold fkv_gemm_q8_0_batched_workspace_size() bytes and be 16-byte aligned:
  * where cols is a multiple of 1024 and every w 16-byte aligned one that is not is
  * FKV_ERR_INVALID "gemm workspace too small" / "gemm workspace must be 16-byte aligned",

@@ -35,7 +35,7 @@ def test_wide_matrices_of_few_rows_take_one_token(tmp_path):
         (16, 14336, 1): (1, 2),
     }
     got = _cuts(tmp_path, list(want))
-    assert dict(zip(want, got)) == want
+    assert {k: c[:2] for k, c in zip(want, got)} == want
 
 
 def test_two_or_four_tokens(tmp_path):
@@ -62,3 +62,28 @@ def test_two_or_four_tokens(tmp_path):
     got = _cuts(tmp_path, list(want))
     assert {k: c[0] for k, c in zip(want, got)} == want
     assert all(c[1] == 1 for c in got)
+
+
+def test_batches_that_the_gemv_takes(tmp_path):
+    """(rows, cols, tokens) -> all workgroups at once. us as a GEMV / on the matrix cores."""
+    want = {
+        (16, 64, 256): 1,        # 3.7 / 5.2
+        (256, 576, 64): 1,       # 4.6 / 6.6
+        (256, 576, 256): 0,      # 10.4 / 6.8
+        (1024, 832, 17): 1,      # 5.0 / 6.1
+        (1024, 4096, 24): 1,     # 9.3 / 10.7
+        (1024, 4096, 32): 0,     # 11.2 / 10.4
+        (1024, 5632, 17): 1,     # 11.6 / 13.1
+        (2048, 2752, 12): 1,     # 8.6 / 8.7
+        (2048, 2752, 16): 0,     # 10.3 / 8.6
+        (4096, 4096, 8): 0,      # 11.5 / 10.2
+        (4096, 4096, 12): 0,     # 15.4 / 10.2: 768 workgroups of four tokens
+        (1024, 4096, 48): 0,     # 13.7 / 10.7
+        (16, 14336, 256): 1,     # 12.2 / 30.6
+        (256, 14336, 24): 1,     # 14.8 / 25.5
+        (1024, 14336, 32): 0,    # 36 / 26.1: two workgroups a CU
+        (1024, 28672, 8): 1,     # 24.8 / 40.6
+        (1024, 28672, 16): 0,    # 45.7 / 40.6
+    }
+    got = _cuts(tmp_path, list(want))
+    assert {k: c[2] for k, c in zip(want, got)} == want

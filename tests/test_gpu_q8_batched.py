@@ -9,8 +9,11 @@ test_cpu_oracle_q8_gemm.py) and fkv_gemm_q8_0's GEMV result, bit for bit, on:
 - several matrices sharing the activation in one launch;
 - non-finite and extreme activations and weight scales;
 - the calls the matrix-core path does not take (fewer than 8 tokens, columns off a
-  multiple of 1024, weights not 16-byte aligned), which run the GEMV;
-and a workspace that is too small is rejected before anything runs.
+  multiple of 64, weights not 4-byte aligned, launches that the GEMV runs at once), which
+  run the GEMV; which of the two a call took is seen by its workspace, which the GEMV
+  leaves alone;
+and a workspace that is too small is rejected before anything runs, or, for widths off a
+multiple of 1024 and weights off 16 bytes, makes the call a GEMV.
 """
 import numpy as np
 import pytest
@@ -52,6 +55,10 @@ def _gemv(w, rows, cols, x):
     (16, 1024, 8), (16, 1024, 16), (33, 1024, 17), (48, 2048, 63), (40, 1024, 64),
     (17, 3072, 65), (64, 2048, 200), (1, 1024, 8), (40, 4096, 37), (4100, 2048, 50),
     (16400, 2048, 40),
+    # on the matrix cores, off and on their tiles of rows and tokens
+    (3073, 1024, 8), (3088, 2048, 9), (1569, 1024, 16), (1456, 3072, 17), (801, 1024, 31),
+    (784, 1024, 32), (736, 4096, 33), (513, 1024, 48), (399, 2048, 63), (385, 1024, 64),
+    (400, 3072, 65), (129, 2048, 200), (4097, 1024, 8), (17, 1024, 770),
 ])
 def test_matches_oracle_and_gemv(rows, cols, n_tokens):
     rng = np.random.default_rng(rows * 131 + cols + n_tokens)
@@ -78,12 +85,12 @@ def test_llama3_8b_shapes_decode_batch(rows, cols):
     _same(got[:, sel], ref.q8_gemm(wr, sel.size, cols, x))
 
 
-def test_several_matrices_one_launch():
+@pytest.mark.parametrize("shapes", [[64, 16, 0, 33], [640, 160, 0, 33]])  # GEMV, matrix cores
+def test_several_matrices_one_launch(shapes):
     """q/k/v of one activation: each output is its own call's, with an empty matrix in
     the middle of the batch."""
     rng = np.random.default_rng(77)
     cols, n_tokens = 2048, 40
-    shapes = [64, 16, 0, 33]
     ws = [_weights(rng, r, cols) if r else np.zeros(0, np.uint8) for r in shapes]
     x = rng.standard_normal((n_tokens, cols)).astype(np.float32)
     ys = _batched(ws, shapes, cols, x)
@@ -92,9 +99,10 @@ def test_several_matrices_one_launch():
             _same(y, ref.q8_gemm(w, r, cols, x))
 
 
-def test_non_finite_and_extreme_inputs():
+@pytest.mark.parametrize("rows", [40, 1301])  # GEMV, matrix cores
+def test_non_finite_and_extreme_inputs(rows):
     rng = np.random.default_rng(12)
-    rows, cols = 40, 1024
+    cols = 1024
     w = _weights(rng, rows, cols, special=True)
     x = rng.standard_normal((20, cols)).astype(np.float32)
     x[0, 3] = np.nan
@@ -135,10 +143,15 @@ def test_large_launches_in_32x32_tiles(rows, cols, n_tokens):
     (50, 576, 33, 12),     # one pair past 16 blocks
     (2048, 5632, 11, 0),
     (16400, 320, 70, 4),   # 32 x 32 tiles, an odd number of pairs
+    # the same widths in launches large enough for the matrix cores
+    (3080, 64, 8, 0), (1569, 192, 16, 4), (1456, 448, 17, 8), (752, 576, 33, 12),
+    (2070, 5632, 11, 0),
+    # 32 x 32 tiles of one and two chunks of blocks, whole and not
+    (8200, 64, 70, 12), (8200, 128, 70, 8), (8200, 192, 70, 0), (8200, 256, 70, 4),
 ])
-def test_columns_off_1024_on_the_matrix_cores(rows, cols, n_tokens, offset):
+def test_columns_off_1024(rows, cols, n_tokens, offset):
     """Any multiple of 64 columns and 4-byte aligned weights, non-finite scales among them;
-    the same bits through the GEMV when there is no workspace."""
+    the same bits through the GEMV when the workspace is too small."""
     import ferrum_amd as fa
     rng = np.random.default_rng(rows + cols + n_tokens)
     w = _weights(rng, rows, cols, special=True)
@@ -153,18 +166,32 @@ def test_columns_off_1024_on_the_matrix_cores(rows, cols, n_tokens, offset):
     _same(_batched([w], [rows], cols, x, offset=offset, workspace=small)[0], want)
 
 
-@pytest.mark.parametrize("rows,cols,n_tokens,offset", [
-    (20, 1024, 7, 0),    # too few tokens: GEMV
-    (20, 544, 30, 0),    # columns off a multiple of 1024: GEMV
-    (20, 1024, 30, 2),   # weights 2 mod 16: GEMV
-    (20, 1024, 30, 8),   # 8 mod 16: GEMV
+@pytest.mark.parametrize("rows,cols,n_tokens,offset,matrix_cores", [
+    (20, 1024, 7, 0, False),       # too few tokens
+    (20, 544, 30, 0, False),       # columns off a multiple of 64
+    (1600, 544, 30, 0, False),
+    (20, 1024, 30, 2, False),      # weights 2 mod 4
+    (1600, 1024, 30, 2, False),
+    (20, 1024, 30, 8, False),      # the GEMV's workgroups all at once
+    (1600, 1024, 30, 8, True),
+    (3072, 1024, 8, 0, False),     # 768 of them, three a CU
+    (3073, 1024, 8, 0, True),      # and one more of rows
+    (48, 576, 510, 4, False),      # 765 in 255 slices of tokens
+    (48, 576, 513, 4, True),
+    (256, 14336, 64, 0, False),    # two of them fill a CU's LDS: 512
+    (256, 14336, 65, 0, True),
 ])
-def test_calls_the_matrix_cores_do_not_take(rows, cols, n_tokens, offset):
+def test_which_calls_the_matrix_cores_take(rows, cols, n_tokens, offset, matrix_cores):
+    import torch
+    import ferrum_amd as fa
     rng = np.random.default_rng(rows + cols + n_tokens + offset)
     w = _weights(rng, rows, cols)
     x = rng.standard_normal((n_tokens, cols)).astype(np.float32)
-    got, = _batched([w], [rows], cols, x, offset=offset)
+    size = max(fa.gemm_q8_0_batched_workspace_bytes(cols, n_tokens), 1 << 20)
+    ws = torch.full((size,), 0x5a, dtype=torch.uint8, device="cuda")
+    got, = _batched([w], [rows], cols, x, offset=offset, workspace=ws)
     _same(got, ref.q8_gemm(w, rows, cols, x))
+    assert bool((ws != 0x5a).any()) == matrix_cores
 
 
 def test_workspace_size_and_rejection():
@@ -188,22 +215,25 @@ def test_workspace_size_and_rejection():
 @pytest.mark.parametrize("case", range(20))
 def test_randomized_batches_against_oracle_and_gemv(case):
     """Seeded random launches: 1 to 4 matrices (an empty one possible) sharing an
-    activation, row counts from 1 to ~5,000 (all three kernel instances: 16-block chunks,
-    32-block chunks with and without the producer wave), columns 1,024 to 6,144, 8 to 150
-    tokens with activation rows of widely different scales; every output against the GEMV
-    bit for bit and a sample of rows against the oracle bit for bit."""
+    activation, row counts from 1 to ~5,000, columns 64 to 6,144 in multiples of 64, weights
+    at 0, 4, 8 or 12 mod 16, 8 to 150 tokens with activation rows of widely different
+    scales; every output against the GEMV bit for bit and a sample of rows against the
+    oracle bit for bit."""
     rng = np.random.default_rng(4000 + case)
-    cols = int(rng.choice([1024, 2048, 3072, 4096, 6144]))
+    cols = int(rng.choice([1024, 2048, 3072, 4096, 6144]) if case % 2 else 64 * rng.integers(1, 97))
+    offset = int(rng.choice([0, 4, 8, 12]))
     n_tokens = int(rng.integers(8, 151))
     nm = int(rng.integers(1, 5))
     rows = [int(rng.choice([0, 1, 15, 16, 17, int(rng.integers(1, 300)), int(rng.integers(300, 5000))]))
             for _ in range(nm)]
     if not any(rows):
         rows[0] = 33
+    if case % 4:  # three in four past the launches that run as a GEMV
+        rows[-1] += 16 * (1664 // n_tokens)
     ws = [_weights(rng, r, cols) if r else np.zeros(0, np.uint8) for r in rows]
     x = (rng.standard_normal((n_tokens, cols)) *
          rng.choice([1e-3, 1.0, 50.0], (n_tokens, 1))).astype(np.float32)
-    ys = _batched(ws, rows, cols, x)
+    ys = _batched(ws, rows, cols, x, offset=offset)
     for r, w, y in zip(rows, ws, ys):
         if not r:
             continue
