@@ -25,6 +25,7 @@
 // a SIMD take 217 cycles a block together; the clock is 1.6-1.8 GHz under that load.
 #include "fkv_device.h"
 #include "fkv_gemm_at.h"
+#include "fkv_gemm_plan.h"
 #include "fkv_gemv_plan.h"
 #include "fkv_q8_act.h"
 
@@ -42,7 +43,7 @@ typedef float f32x32 __attribute__((ext_vector_type(32)));
 
 constexpr uint32_t kQ8Bytes = 34;
 static_assert(gemm_at::kPairBytes == 2 * kQ8Bytes, "a pair of blocks");
-constexpr uint32_t kTileRows = 64;      // weight rows of a workgroup
+constexpr uint32_t kTileRows = kGemmTileRows;
 [[maybe_unused]] constexpr uint32_t kMagicBits = 0x4b400000u;
 [[maybe_unused]] constexpr float kMagic = 12582912.0f;    // 1.5 * 2^23
 
@@ -56,7 +57,7 @@ __host__ __device__ constexpr uint64_t act_quant_bytes(uint32_t n_tiles, uint32_
   return (uint64_t)n_tiles * nb * 512u;
 }
 
-constexpr uint32_t kActThreads = 64;
+constexpr uint32_t kActThreads = kGemmActThreads;
 
 template <bool kPairs>
 __global__ __launch_bounds__(kActThreads) void q8_act_tile_kernel(const float* __restrict__ x,
@@ -583,27 +584,13 @@ bool gemm_mfma_needs_workspace(const GemvBatch& b, uint32_t cols) {
 bool gemm_mfma_pays(const GemvBatch& b, uint32_t cols, uint32_t n_tokens) {
   uint32_t n_wg = 0;
   for (uint32_t m = 0; m < b.n; ++m) n_wg += (b.m[m].rows + kGemvRowsPerWg - 1u) / kGemvRowsPerWg;
-  return !gemv_runs_at_once(n_tokens, cols, n_wg);
+  return !gemv_runs_at_once(n_tokens, cols, n_wg) &&
+         gemm_act_threads(cols, n_tokens) <= kMaxGridThreads;
 }
 
 uint64_t gemm_mfma_workspace_bytes(uint32_t cols, uint32_t n_tokens) {
   const uint32_t n_tiles = (n_tokens + 15u) / 16u, nb = cols / 32u;
   return act_quant_bytes(n_tiles, nb) + (uint64_t)n_tiles * nb * 16u * 4u;
-}
-
-// A workgroup of the 64 x 64 kernel takes about as long alone on its CU as with two others
-// (4,096 columns: 25 us at one a CU, 34 us at three), so it wins once every CU has one:
-// at 256 workgroups and 4,096 x 4,096 weights 28.1 us against 30.5 for 16 x 16 tiles (256
-// tokens), at 192 27.0 against 24.3 (192 tokens); 2,048 and 14,336 columns turn at the same
-// count (17.4 / 19.4 and 77.5 / 85.7 us at 256). And the tokens have to use more than half
-// of its 64: 28,672 rows, 32 tokens 48.5 us against 47.2, 64 tokens 50 against 69.
-constexpr uint64_t kTileMinWgs = 256;
-constexpr uint32_t kTileMinTokens = 33;
-static bool gemm_tile_fills(const GemvBatch& b, uint32_t n_tokens) {
-  uint64_t row_tiles = 0;
-  for (uint32_t m = 0; m < b.n; ++m) row_tiles += (b.m[m].rows + kTileRows - 1u) / kTileRows;
-  const uint64_t wgs = row_tiles * ((n_tokens + 63u) / 64u);
-  return n_tokens >= kTileMinTokens && wgs >= kTileMinWgs && wgs < (1ull << 30);
 }
 
 template <int W>
@@ -616,7 +603,9 @@ static void launch_rows(const GemvBatch& b, uint32_t row_tiles, uint32_t cols, u
 
 hipError_t launch_gemm_q8_mfma(GemvBatch b, uint32_t cols, const float* x, uint32_t n_tokens,
                                void* workspace, hipStream_t s) {
-  const bool tiles = gemm_tile_fills(b, n_tokens);
+  uint64_t tile_rows = 0;
+  for (uint32_t m = 0; m < b.n; ++m) tile_rows += (b.m[m].rows + kTileRows - 1u) / kTileRows;
+  const bool tiles = gemm_tile_fills(tile_rows, n_tokens);
   const uint32_t row_tile = tiles ? kTileRows : kRowTile;
   uint32_t row_tiles = 0;
   for (uint32_t m = 0; m < b.n; ++m) {
@@ -625,8 +614,7 @@ hipError_t launch_gemm_q8_mfma(GemvBatch b, uint32_t cols, const float* x, uint3
   }
   for (uint32_t m = b.n; m < (uint32_t)kGemvMaxMats; ++m) b.m[m] = b.m[0];
   const uint32_t n_tiles = (n_tokens + 15u) / 16u, token_tiles = (n_tiles + 3u) / 4u;
-  const uint64_t items = (uint64_t)n_tiles * 16u * (cols / 8u);
-  const uint32_t act_grid = (uint32_t)((items + kActThreads - 1u) / kActThreads);
+  const uint32_t act_grid = (uint32_t)(gemm_act_threads(cols, n_tokens) / kActThreads);
   uint8_t* wsp = (uint8_t*)workspace;
   if (tiles)
     q8_act_tile_kernel<false><<<act_grid, kActThreads, 0, s>>>(x, cols, n_tokens, n_tiles, wsp);
@@ -635,7 +623,7 @@ hipError_t launch_gemm_q8_mfma(GemvBatch b, uint32_t cols, const float* x, uint3
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   if (tiles)
-    gemm_q8_tile_kernel<<<(row_tiles + 7u) / 8u * 8u * token_tiles, 256, 0, s>>>(
+    gemm_q8_tile_kernel<<<(uint32_t)gemm_tile_wgs(row_tiles, n_tokens), kGemmTileThreads, 0, s>>>(
         b, cols, n_tokens, n_tiles, row_tiles, token_tiles, wsp);
   else if (n_tiles == 1u)
     launch_rows<1>(b, row_tiles, cols, n_tokens, n_tiles, wsp, s);

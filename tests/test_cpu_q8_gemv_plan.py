@@ -1,5 +1,6 @@
-"""CPU: how a Q8_0 GEMV launch is cut up (ferrum_amd/csrc/fkv_gemv_plan.h) at sizes whose
-better cut was measured; the cut changes no result, so only its choice is checked."""
+"""CPU: how a Q8_0 GEMV launch is cut up (ferrum_amd/csrc/fkv_gemv_plan.h) and which kernel
+a batched GEMM runs (fkv_gemm_plan.h), at sizes where both sides were measured or a limit
+lies; neither changes a result, so only the choice is checked."""
 import os
 import shutil
 import subprocess
@@ -10,10 +11,10 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 pytestmark = pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
 
 
-def _cuts(tmp_path, sizes):
-    exe = tmp_path / "gemv_plan_print"
+def _cuts(tmp_path, sizes, program="gemv_plan_print"):
+    exe = tmp_path / program
     subprocess.run(["g++", "-O2", "-std=c++17", "-Wall", "-o", str(exe),
-                    os.path.join(HERE, "gemm", "gemv_plan_print.cpp")], check=True)
+                    os.path.join(HERE, "gemm", program + ".cpp")], check=True)
     text = "".join("%d %d %d\n" % s for s in sizes)
     out = subprocess.run([str(exe)], input=text, capture_output=True, text=True, check=True)
     return [tuple(map(int, line.split())) for line in out.stdout.splitlines()]
@@ -87,3 +88,24 @@ def test_batches_that_the_gemv_takes(tmp_path):
     }
     got = _cuts(tmp_path, list(want))
     assert {k: c[2] for k, c in zip(want, got)} == want
+
+
+def test_launches_stay_within_one_grid(tmp_path):
+    """(row tiles, cols, tokens) -> 64 x 64 tiles? Sizes up to the card's memory and past it."""
+    want = {
+        (448, 4096, 64): 1,
+        (448, 4096, 32): 0,                   # half a tile's tokens or fewer
+        (255, 4096, 64): 0,
+        (1, 64, 64 * (1 << 21) - 64): 1,      # 2^24 - 8 workgroups of 256
+        (1, 64, 64 * (1 << 21)): 0,           # 2^32 threads
+        (2, 64, 1 << 30): 0,
+        (2048, 64, 64 * 8191): 1,
+        (2048, 64, 64 * 8192): 0,
+    }
+    got = _cuts(tmp_path, list(want), "gemm_plan_print")
+    assert {k: g[0] for k, g in zip(want, got)} == want
+    for (row_tiles, cols, tokens), (tiles, threads, act) in zip(want, got):
+        assert not tiles or threads < 2 ** 32
+        assert act == -(-tokens // 16) * 16 * cols // 8
+    (_, _, past), = _cuts(tmp_path, [(1, 5632, 6_200_000)], "gemm_plan_print")
+    assert past > 2 ** 32 - 1                 # the caller then runs the GEMV
