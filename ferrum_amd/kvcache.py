@@ -18,13 +18,26 @@ from typing import Optional, Sequence
 
 import numpy as np
 
-try:
-    import torch
-except ImportError:  # the host-only surface works without it
-    torch = None
-
 from . import _lib
 from .errors import check
+
+_torch_loaded = None
+_raw_stream = None  # torch's (current raw stream of a device, current device) functions
+
+
+def _torch():
+    """torch, imported by the first device call: the host-only surface neither needs it nor
+    waits for it (2 s), and a device call without it is its ImportError. A global read
+    afterwards, as an import statement is 0.2 us in every call."""
+    global _torch_loaded, _raw_stream
+    if _torch_loaded is None:
+        import torch
+        get = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+        device = getattr(torch._C, "_cuda_getDevice", None)
+        if get is not None and device is not None:
+            _raw_stream = get, device
+        _torch_loaded = torch
+    return _torch_loaded
 
 __all__ = ["KvPoolConfig", "PreallocatedKvPool", "PagedConfig", "PagedKvPool",
            "default_scale"]
@@ -150,11 +163,13 @@ class PagedConfig:
 
 def _stream_ptr(stream) -> int:
     """The HIP stream handle; None: the current device's current stream. Asked of torch's
-    C layer where CUDA is initialised: torch.cuda.current_stream() builds a Stream object
-    (3.0 us against 0.4), in a call whose launches take 6."""
+    C layer where CUDA is initialised and that layer has it: torch.cuda.current_stream()
+    builds a Stream object (3.0 us against 0.4), in a call whose launches take 6."""
     if stream is None:
-        if torch.cuda.is_initialized():
-            return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+        torch = _torch()
+        if _raw_stream is not None and torch.cuda.is_initialized():
+            get, device = _raw_stream
+            return get(device())
         return torch.cuda.current_stream().cuda_stream
     if isinstance(stream, int):
         return stream
@@ -162,7 +177,7 @@ def _stream_ptr(stream) -> int:
 
 
 def _dev(t, dtype, name):
-    if not isinstance(t, torch.Tensor) or not t.is_cuda:
+    if not isinstance(t, _torch_loaded.Tensor) or not t.is_cuda:
         raise TypeError(f"{name} must be a device tensor")
     if t.dtype != dtype:
         raise TypeError(f"{name} must be {dtype}, got {t.dtype}")
@@ -266,6 +281,7 @@ class PagedKvPool:
 
     # -- device operations --------------------------------------------------
     def append(self, layer: int, k, v, slot_mapping, stream=None) -> None:
+        torch = _torch()
         n = slot_mapping.numel()
         row = self.config.n_kv_heads * self.config.head_dim
         if k.numel() != n * row or v.numel() != n * row:
@@ -277,6 +293,7 @@ class PagedKvPool:
 
     def gather_slots(self, layer: int, slot_mapping, out_k, out_v,
                      fmt: int = _lib.GATHER_F32, stream=None) -> None:
+        torch = _torch()
         check(self._lib.fkv_gather_slots(self._h, layer,
                                          _dev(slot_mapping, torch.int64, "slot_mapping"),
                                          slot_mapping.numel(), fmt,
@@ -284,6 +301,7 @@ class PagedKvPool:
 
     def gather_tables(self, layer: int, block_tables, ctx_lens, out_offsets, max_ctx_len: int,
                       out_k, out_v, fmt: int = _lib.GATHER_F32, stream=None) -> None:
+        torch = _torch()
         n_seqs, max_blocks = block_tables.shape
         check(self._lib.fkv_gather_tables(self._h, layer,
                                           _dev(block_tables, torch.int32, "block_tables"),
@@ -293,6 +311,7 @@ class PagedKvPool:
                                           _stream_ptr(stream)))
 
     def copy_blocks(self, pairs, stream=None) -> None:
+        torch = _torch()
         check(self._lib.fkv_copy_blocks(self._h, _dev(pairs, torch.int64, "pairs"),
                                         pairs.shape[0], _stream_ptr(stream)))
 
@@ -321,6 +340,7 @@ class PagedKvPool:
                          scale: Optional[float] = None, workspace=None, stream=None) -> None:
         """q, out: float32 [n_seqs, n_heads, head_dim]; block_tables int32 [n_seqs, max_blocks];
         ctx_lens int32 [n_seqs]."""
+        torch = _torch()
         n_seqs, n_heads, d = q.shape
         if d != self.config.head_dim or tuple(out.shape) != tuple(q.shape):
             raise ValueError("q/out must be [n_seqs, n_heads, head_dim]")
@@ -348,6 +368,7 @@ class PagedKvPool:
         """One decode step of one layer (llama.rs:218-247): store k_new/v_new (float32
         [n_seqs, n_kv_heads, head_dim]) at position ctx_lens[s] - 1 through the block
         tables, then decode attention over ctx_lens[s] positions."""
+        torch = _torch()
         n_seqs, n_heads, d = q.shape
         if d != self.config.head_dim or tuple(out.shape) != tuple(q.shape):
             raise ValueError("q/out must be [n_seqs, n_heads, head_dim]")
@@ -380,6 +401,7 @@ class PagedKvPool:
         """append_decode_attention with no workspace and no allocation: the split
         partials go to the library's static per-GPU scratch (STATIC_SCRATCH_BYTES).
         Calls that overlap on one GPU race on it; a step needing more is InvalidRequest."""
+        torch = _torch()
         n_seqs, n_heads, d = q.shape
         if d != self.config.head_dim or tuple(out.shape) != tuple(q.shape):
             raise ValueError("q/out must be [n_seqs, n_heads, head_dim]")
@@ -405,6 +427,7 @@ class PagedKvPool:
         each sequence's q and k_new are rotated at position ctx_lens[s] - 1 (dims
         (2i, 2i+1) below rope_dim, angle pos / theta^(2i/rope_dim); scalar.rs:167-189)
         before the append and the attention. q is not written back."""
+        torch = _torch()
         n_seqs, n_heads, d = q.shape
         if d != self.config.head_dim or tuple(out.shape) != tuple(q.shape):
             raise ValueError("q/out must be [n_seqs, n_heads, head_dim]")
@@ -447,6 +470,7 @@ class PagedKvPool:
         ctx_lens[s] context, each attending causally (crates/model/src/llama.rs:363-378).
         workspace: device scratch for the key-range pieces (allocated here when None);
         split=False passes none, so every workgroup reads its whole key range."""
+        torch = _torch()
         rows, n_heads, d = q.shape
         if d != self.config.head_dim or tuple(out.shape) != tuple(q.shape):
             raise ValueError("q/out must be [rows, n_heads, head_dim]")

@@ -17,14 +17,9 @@ from __future__ import annotations
 
 import ctypes
 
-try:
-    import torch
-except ImportError:
-    torch = None
-
-from . import _lib
+from . import _lib, kvcache
 from .errors import check
-from .kvcache import _stream_ptr
+from .kvcache import _stream_ptr, _torch
 
 __all__ = ["Q8_0_BLOCK", "Q8_0_BLOCK_BYTES", "gemv_q8_0", "gemm_q8_0", "gemm_q8_0_multi",
            "gemm_q8_0_batched", "gemm_q8_0_batched_workspace_bytes", "q8_0_row_bytes"]
@@ -39,7 +34,7 @@ def q8_0_row_bytes(cols: int) -> int:
 
 
 def _dev_any(t, dtype, name):
-    if not isinstance(t, torch.Tensor) or not t.is_cuda:
+    if not isinstance(t, kvcache._torch_loaded.Tensor) or not t.is_cuda:
         raise TypeError(f"{name} must be a device tensor")
     if t.dtype != dtype:
         raise TypeError(f"{name} must be {dtype}, got {t.dtype}")
@@ -50,6 +45,7 @@ def _dev_any(t, dtype, name):
 
 def gemv_q8_0(w, rows: int, cols: int, x, y, stream=None) -> None:
     """Kernels::gemv(DType::Q8_0, w, rows, cols, x, y): y[r] for one activation row."""
+    torch = _torch()
     wp, wn = _dev_any(w, torch.uint8, "w")
     xp, xn = _dev_any(x, torch.float32, "x")
     yp, yn = _dev_any(y, torch.float32, "y")
@@ -59,6 +55,7 @@ def gemv_q8_0(w, rows: int, cols: int, x, y, stream=None) -> None:
 def gemm_q8_0(w, rows: int, cols: int, x, n_tokens: int, y, stream=None) -> None:
     """Kernels::gemm(GemmArgs { dtype: Q8_0, w, rows, cols, x, n_tokens, y }):
     y[t * rows + r], each token as gemv_q8_0 of x[t]."""
+    torch = _torch()
     wp, wn = _dev_any(w, torch.uint8, "w")
     xp, xn = _dev_any(x, torch.float32, "x")
     yp, yn = _dev_any(y, torch.float32, "y")
@@ -69,6 +66,7 @@ def gemm_q8_0(w, rows: int, cols: int, x, n_tokens: int, y, stream=None) -> None
 def gemm_q8_0_multi(ws, rows, cols: int, x, n_tokens: int, ys, stream=None) -> None:
     """gemm_q8_0 of up to 4 matrices that take the same x (q/k/v, gate/up) in one launch;
     ys[m] equals gemm_q8_0(ws[m], rows[m], cols, x, n_tokens, ys[m]) bit for bit."""
+    torch = _torch()
     n = len(ws)
     if len(rows) != n or len(ys) != n:
         raise ValueError("ws, rows and ys must have one entry per matrix")
@@ -94,6 +92,7 @@ def gemm_q8_0_batched(ws, rows, cols: int, x, n_tokens: int, ys, workspace=None,
     """gemm_q8_0_multi on the matrix cores for batches (n_tokens >= 8, cols a multiple of
     64, 4-byte aligned weights; otherwise the GEMV), bit-identical. `workspace`: a
     device uint8 tensor of gemm_q8_0_batched_workspace_bytes (allocated here when None)."""
+    torch = _torch()
     n = len(ws)
     if len(rows) != n or len(ys) != n:
         raise ValueError("ws, rows and ys must have one entry per matrix")
