@@ -345,6 +345,27 @@ __global__ void __launch_bounds__(256) append_q8_kernel(Geom g, uint32_t layer,
   }
 }
 
+// Lanes 0 .. 15 hold the slots of a window's tokens: -1 where a later lane names the same
+// slot. Slots that rise from lane to lane hold none, so most windows take one comparison.
+template <int N>
+__device__ __forceinline__ bool slot_repeats(int64_t sl) {
+  if constexpr (N == 16) {
+    return false;
+  } else {
+    const int lo = __builtin_amdgcn_update_dpp(-1, (int)(uint32_t)sl, 0x100 + N, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(-1, (int)(sl >> 32), 0x100 + N, 0xf, 0xf, false);
+    const bool same = lo == (int)(uint32_t)sl && hi == (int)(sl >> 32);  // row_shl:N
+    return same | slot_repeats<N + 1>(sl);
+  }
+}
+__device__ __forceinline__ int64_t drop_repeated_slot(int64_t sl) {
+  const int lo = __builtin_amdgcn_update_dpp(-1, (int)(uint32_t)sl, 0x101, 0xf, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(-1, (int)(sl >> 32), 0x101, 0xf, 0xf, false);
+  const int64_t next = ((int64_t)hi << 32) | (uint32_t)lo;
+  if (__ballot(threadIdx.x % 16u != 15u && sl >= next) == 0) return sl;
+  return sl >= 0 && slot_repeats<1>(sl) ? -1 : sl;
+}
+
 // Q8_0 storage, head_dim 64 or 128, 16-byte aligned k/v: one workgroup per 16
 // consecutive tokens x 128 / D KV heads. Bound by HBM: it reads 8 bytes a K/V element
 // pair and writes 2 and a scale's share. So loads are coalesced and many: thread
@@ -359,6 +380,8 @@ __global__ void __launch_bounds__(256) append_q8_kernel(Geom g, uint32_t layer,
 // segment is the whole group and by single bytes otherwise.
 // Measured with 8 KV heads of 128 dims, 8,192 tokens (84 MB): 30.6 -> 25.5 us, 3.3 TB/s;
 // 24,000 tokens 54.2 -> 52.7 (4.7 TB/s).
+// A slot named twice in a window goes to the last of its tokens (drop_repeated_slot): its
+// scales and quants are stored by different waves.
 template <int D>
 __global__ void __launch_bounds__(256) append_q8_tile_kernel(Geom g, uint32_t layer,
                                                              const float* __restrict__ k,
@@ -391,7 +414,7 @@ __global__ void __launch_bounds__(256) append_q8_tile_kernel(Geom g, uint32_t la
       raise_fault(g.fault, kFaultSlot);
       sl = -1;
     }
-    s_slot[threadIdx.x] = sl;
+    s_slot[threadIdx.x] = drop_repeated_slot(sl);
   }
   __syncthreads();
 

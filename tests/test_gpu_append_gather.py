@@ -131,6 +131,31 @@ def test_append_q8_windows_bit_exact(d, hkv, block_size):
     assert pool.take_fault_flags() == 0
 
 
+@pytest.mark.parametrize("d,hkv", [(64, 3), (128, 2)])
+def test_append_q8_slot_named_twice(d, hkv):
+    """A slot that two or more tokens of one window of 16 name holds the last of them, its
+    scales and quants alike (next to each other, across 4-token groups, all sixteen, and
+    around slots that are skipped)."""
+    from oracle import ref
+    rng = np.random.default_rng(d)
+    windows = [[0, 1, 2, 3, 4, 5, 3, 7, 8, 9, 10, 11, 3, 13, 14, 15],
+               [16, 16] + [18] * 3 + list(range(21, 32)),
+               [32] * 16,
+               [-1, 50, -1, -1, 50, 51, 52, 53, 60, 59, 58, 57, 50, -1, 60, -1],
+               list(range(79, 71, -1)) + list(range(79, 71, -1)),
+               [80, 95, 80]]
+    slots = np.concatenate(windows).astype(np.int64)
+    k = rng.standard_normal((slots.size, hkv, d), dtype=np.float32)
+    v = rng.standard_normal((slots.size, hkv, d), dtype=np.float32)
+    pool, layout = make_pools(1, hkv, d, 8, dtype=8)
+    pool.fill(0x5a)
+    want = np.full(layout.pool_bytes, 0x5a, np.uint8)
+    pool.append(0, to_dev(k), to_dev(v), to_dev(slots))
+    ref.append(layout, want, 0, k, v, slots)
+    mism = np.flatnonzero(pool.read() != want)
+    assert mism.size == 0, f"{mism.size} bytes differ, first at {mism[:4]}"
+
+
 @pytest.mark.parametrize("dtype,d", [(0, 128), (1, 128), (1, 64), (8, 64), (0, 4), (1, 12)])
 def test_append_gather_roundtrip_scattered(dtype, d):
     """Append through a scattered slot mapping (with -1 padding), gather back by
