@@ -343,30 +343,28 @@ __global__ __launch_bounds__(256, 2) void gemm_q8_tile_kernel(const GemvBatch ba
 // through a ring of chunks in LDS by direct loads; the computing waves load the
 // activation, which the L2 holds, four groups of blocks ahead into registers. Loads retire
 // in order, so with the weight loads in the computing waves each activation load would
-// wait for HBM. A short ring of small chunks leaves room for 4 to 8 workgroups a CU and
-// little to fill before the first block: 3 chunks of 8 blocks against 6 of 16, us at 16
-// tokens: q/k/v 11.5 / 13.5, attn_output 10.5 / 11.5, gate/up 38.4 / 44.5, down 24.9 / 26.3.
-// Against the kernel before (one variant with and one without such a wave, weights
-// through registers, four VALU instructions): 16 tokens 14.9, 12.6, 39.8, 26.4; 64 tokens
-// q/k/v 18.4 -> 15.9, attn_output 13.6 -> 12.9, down 32.6 -> 31.8.
-[[maybe_unused]] constexpr uint32_t kRing = 3;
+// wait for HBM. Against the kernel before (one variant with and one without such a wave,
+// weights through registers, four VALU instructions), us with weights from HBM, 16 tokens:
+// q/k/v 14.3 -> 12.1, attn_output 12.9 -> 11.4, gate/up 40.8 -> 40.0, down 29.3 -> 26.4; 64
+// tokens: 19.0 -> 15.9, 14.5 -> 13.3, gate/up in 64 x 64 tiles, 35.0 -> 30.1.
+// Chunk, ring and the groups loaded ahead are the launch's (gemm_rows_cut).
 [[maybe_unused]] constexpr uint32_t kGroup = 4;    // blocks of a step
-constexpr uint32_t kPairs = 4;    // pairs of blocks of a chunk
-[[maybe_unused]] constexpr int kGroups = 2;        // and its groups
-constexpr uint32_t kRowTile = 16;
+constexpr uint32_t kRowTile = kGemmRowTile;
 
+template <uint32_t kPairs>
 struct RowChunk {
   uint4 wq[kPairs][kRowTile][4];   // as Chunk's
   uint32_t we[kPairs][kRowTile];
 };
 
 // kTail: columns not a multiple of 512. The blocks that fill the row's last 16 up get
-// scales of zero (the next row's weights may stand there), so they add +0.
-// W computing waves, a 16-token tile each.
-template <int W, bool kTail>
-__global__ __launch_bounds__((W + 1) * 64, 4) void gemm_q8_rows_kernel(const GemvBatch bat, uint32_t cols,
-                                                              uint32_t n_tokens, uint32_t n_tiles,
-                                                              const uint8_t* __restrict__ ws) {
+// scales of zero (the row's last pair is read for them), so they add +0.
+// W computing waves, a 16-token tile each. Chunks of kPairs pairs, a ring of kRing; kAhead
+// groups of activation in registers.
+template <int W, bool kTail, uint32_t kPairs, uint32_t kRing, int kAhead>
+__global__ __launch_bounds__((W + 1) * 64, kAhead == 4 ? 4 : 2) void gemm_q8_rows_kernel(
+    const GemvBatch bat, uint32_t cols, uint32_t n_tokens, uint32_t n_tiles,
+    const uint8_t* __restrict__ ws) {
 #ifdef __HIP_DEVICE_COMPILE__  // the host pass needs the kernel's stub only
   uint32_t mi = 0;
 #pragma unroll
@@ -377,13 +375,17 @@ __global__ __launch_bounds__((W + 1) * 64, 4) void gemm_q8_rows_kernel(const Gem
   const uint32_t nb = cols / 32u, np = nb / 2u;
   // groups, runs of 4 groups
   const uint32_t ng = (nb + kGroup - 1u) / kGroup, n4 = (ng + 3u) / 4u;
-  // barriers: one a chunk, and two chunks read past the row's end (up to 3 groups ahead)
-  const uint32_t n_bar = 2u + n4 * 2u;
+  constexpr int kGroups = (int)kPairs / 2;  // of a chunk
+  static_assert(kGroups == 2 || kGroups == 4, "whole chunks a run of 4 groups");
+  static_assert(kAhead == 4 || kAhead == 8, "whole runs a turn of the registers");
+  // barriers: one a chunk, and the chunks read past the row's end (up to 3 groups ahead)
+  const uint32_t n_bar = (kGroups == 2 ? 2u : 1u) + n4 * (4u / (uint32_t)kGroups);
   const uint32_t lane = threadIdx.x & 63u;
   const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const uint32_t c = lane & 15u, grp = lane >> 4;
 
-  __shared__ RowChunk ring[kRing];
+  using Rows = RowChunk<kPairs>;
+  __shared__ Rows ring[kRing];
   auto barrier = [] {
     __asm__ volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();
@@ -399,23 +401,25 @@ __global__ __launch_bounds__((W + 1) * 64, 4) void gemm_q8_rows_kernel(const Gem
     const uint32_t w_off = gemm_at::rows_weights(lane, last_row, (uint32_t)row_bytes);
     const uint32_t e_off = gemm_at::rows_dwords8(lane, last_row, (uint32_t)row_bytes);
     auto stage = [&](uint32_t k) __attribute__((always_inline)) {
-      RowChunk& L = ring[k % kRing];
+      Rows& L = ring[k % kRing];
 #pragma unroll
       for (uint32_t i = 0; i < kPairs; ++i)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(
             rw, (__attribute__((address_space(3))) void*)&L.wq[i][0][0], 16, w_off,
             (int)gemm_at::pair(k * kPairs + i, np), 0, 0);
-      static_assert(kPairs == 4u, "one load holds the pairs' dwords 8");
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          rw, (__attribute__((address_space(3))) void*)&L.we[0][0], 4,
-          e_off + gemm_at::pair(k * kPairs + grp, np), 0, 0, 0);
+#pragma unroll
+      for (uint32_t i = 0; i < kPairs; i += 4u)  // 4 pairs' dwords 8
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(
+            rw, (__attribute__((address_space(3))) void*)&L.we[i][0], 4,
+            e_off + gemm_at::pair(k * kPairs + i + grp, np), 0, 0, 0);
     };
     for (uint32_t k = 0; k + 1u < kRing; ++k) stage(k);
     // Before barrier k: chunk k has landed (kRing - 2 later ones may be in flight). After
     // it every wave is done with chunk k - 1, whose buffer takes chunk k - 1 + kRing.
-    static_assert((kPairs + 1u) * (kRing - 2u) == 5u, "the wait below");
+    constexpr uint32_t kInFlight = (kPairs + kPairs / 4u) * (kRing - 2u);
+    static_assert(kInFlight < 16u, "the wait's field");
     for (uint32_t k = 0; k < n_bar; ++k) {
-      __builtin_amdgcn_s_waitcnt(0x0f75);  // vmcnt(5)
+      __builtin_amdgcn_s_waitcnt(0x0f70 | kInFlight);  // vmcnt
       barrier();
       stage(k + kRing - 1u);
     }
@@ -436,8 +440,8 @@ __global__ __launch_bounds__((W + 1) * 64, 4) void gemm_q8_rows_kernel(const Gem
       lds_source(ws + act_quant_bytes(n_tiles, nb) + (uint64_t)tt * nb * 64u, nb * 64u);
   const int32_t blocks_left = (int32_t)nb - (int32_t)grp;
   const uint32_t xq_off = lane * 16u;
-  uint4 xq[4][2];
-  uint32_t xs[4];
+  uint4 xq[kAhead][2];
+  uint32_t xs[kAhead];
   auto load_x = [&](uint32_t g, int slot) __attribute__((always_inline)) {
     xq[slot][0] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rq, xq_off, gemm_at::rows_quants(2u * g, np), 0));
     xq[slot][1] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rq, xq_off, gemm_at::rows_quants(2u * g + 1u, np), 0));
@@ -449,7 +453,7 @@ __global__ __launch_bounds__((W + 1) * 64, 4) void gemm_q8_rows_kernel(const Gem
   // pairs' dwords 8 and the scale of block grp.
   const uint32_t f = c / 4u;
   const uint32_t o_even = c * 64u + ((grp / 2u) ^ f) * 16u + (grp % 2u) * 8u, o_odd = o_even ^ 32u;
-  const uint32_t o_we = (uint32_t)offsetof(RowChunk, we) + c * 4u;
+  const uint32_t o_we = (uint32_t)offsetof(Rows, we) + c * 4u;
   const bool s_odd = grp % 2u != 0u;
   const uint32_t o_s = s_odd ? o_we + (grp / 2u) * 64u + 2u : (grp / 2u) * 1024u + c * 64u + f * 16u;
   const uint32_t s_step = s_odd ? 128u : 2048u;  // a group on
@@ -513,30 +517,31 @@ __global__ __launch_bounds__((W + 1) * 64, 4) void gemm_q8_rows_kernel(const Gem
   };
 
 #pragma unroll
-  for (int j = 0; j < 4; ++j) load_x((uint32_t)j, j);
+  for (int j = 0; j < kAhead; ++j) load_x((uint32_t)j, j);
   barrier();  // chunk 0
   read_w(0);
   dots(0, 0);
   dots(1, 0);
   scales(0, 0);
-  load_x(4, 0);
+  load_x((uint32_t)kAhead, 0);
   read_w(1);
   uint32_t base = 0;
   auto next_chunk = [&]() __attribute__((always_inline)) {
     __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this wave has read the last one
     barrier();
-    base = base + sizeof(RowChunk) < sizeof(ring) ? base + (uint32_t)sizeof(RowChunk) : 0u;
+    base = base + sizeof(Rows) < sizeof(ring) ? base + (uint32_t)sizeof(Rows) : 0u;
     at_chunk(base);
   };
-  next_chunk();
+  if (kGroups == 2) next_chunk();
   read_w(2);
-  for (uint32_t k = 0; k < n4; ++k) {
+  for (uint32_t k = 0; k < n4; k += (uint32_t)kAhead / 4u) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < kAhead; ++j) {
+      if (j == 4 && k + 1u >= n4) break;
       // Group g, while group g + 1's products go through the matrix cores from the operands
-      // in registers, which then take group g + 3's weights and g + 5's activation.
+      // in registers, which then take group g + 3's weights and g + 1 + kAhead's activation.
       const uint32_t g = 4u * k + (uint32_t)j;
-      const int n = (j + 1) % 4;
+      const int n = (j + 1) % kAhead;
       __builtin_amdgcn_sched_barrier(0);
       products(0);
       add();
@@ -549,7 +554,7 @@ __global__ __launch_bounds__((W + 1) * 64, 4) void gemm_q8_rows_kernel(const Gem
       add();
       __builtin_amdgcn_sched_barrier(0);
       dots(1, n);
-      load_x(g + 5u, n);
+      load_x(g + 1u + (uint32_t)kAhead, n);
       if ((j + 3) % kGroups == 0) next_chunk();
       read_w((j + 3) % 4);
     }
@@ -593,19 +598,41 @@ uint64_t gemm_mfma_workspace_bytes(uint32_t cols, uint32_t n_tokens) {
   return act_quant_bytes(n_tiles, nb) + (uint64_t)n_tiles * nb * 16u * 4u;
 }
 
+template <int W, uint32_t kPairs, uint32_t kRing, int kAhead>
+static void launch_rows_as(const GemvBatch& b, dim3 grid, uint32_t spare_lds, uint32_t cols,
+                           uint32_t n_tokens, uint32_t n_tiles, const uint8_t* ws, hipStream_t s) {
+  const auto kernel = cols % 512u != 0u ? gemm_q8_rows_kernel<W, true, kPairs, kRing, kAhead>
+                                        : gemm_q8_rows_kernel<W, false, kPairs, kRing, kAhead>;
+  kernel<<<grid, (W + 1) * 64, spare_lds, s>>>(b, cols, n_tokens, n_tiles, ws);
+}
 template <int W>
 static void launch_rows(const GemvBatch& b, uint32_t row_tiles, uint32_t cols, uint32_t n_tokens,
-                 uint32_t n_tiles, const uint8_t* ws, hipStream_t s) {
+                        uint32_t n_tiles, const uint8_t* ws, hipStream_t s) {
   const dim3 grid(row_tiles, (n_tiles + W - 1u) / W);
-  const auto kernel = cols % 512u != 0u ? gemm_q8_rows_kernel<W, true> : gemm_q8_rows_kernel<W, false>;
-  kernel<<<grid, (W + 1) * 64, 0, s>>>(b, cols, n_tokens, n_tiles, ws);
+  const GemmRowsCut cut = gemm_rows_cut(W, cols, row_tiles, (uint64_t)grid.x * grid.y);
+  if constexpr (W <= 2) {
+    if (!cut.wide && cut.ahead == 4u)
+      return launch_rows_as<W, 4, 3, 4>(b, grid, cut.spare_lds, cols, n_tokens, n_tiles, ws, s);
+  }
+  if constexpr (W == 1) {
+    launch_rows_as<W, 4, 3, 8>(b, grid, cut.spare_lds, cols, n_tokens, n_tiles, ws, s);
+  } else {
+    if constexpr (W >= 3) {
+      if (cut.ahead == 4u)
+        return launch_rows_as<W, 8, 2, 4>(b, grid, cut.spare_lds, cols, n_tokens, n_tiles, ws, s);
+    }
+    launch_rows_as<W, 8, 2, 8>(b, grid, cut.spare_lds, cols, n_tokens, n_tiles, ws, s);
+  }
 }
 
 hipError_t launch_gemm_q8_mfma(GemvBatch b, uint32_t cols, const float* x, uint32_t n_tokens,
                                void* workspace, hipStream_t s) {
-  uint64_t tile_rows = 0;
-  for (uint32_t m = 0; m < b.n; ++m) tile_rows += (b.m[m].rows + kTileRows - 1u) / kTileRows;
-  const bool tiles = gemm_tile_fills(tile_rows, n_tokens);
+  uint64_t tile_rows = 0, row_tiles_16 = 0;
+  for (uint32_t m = 0; m < b.n; ++m) {
+    tile_rows += (b.m[m].rows + kTileRows - 1u) / kTileRows;
+    row_tiles_16 += (b.m[m].rows + kRowTile - 1u) / kRowTile;
+  }
+  const bool tiles = gemm_tile_wins(tile_rows, row_tiles_16, cols, n_tokens);
   const uint32_t row_tile = tiles ? kTileRows : kRowTile;
   uint32_t row_tiles = 0;
   for (uint32_t m = 0; m < b.n; ++m) {
@@ -625,12 +652,13 @@ hipError_t launch_gemm_q8_mfma(GemvBatch b, uint32_t cols, const float* x, uint3
   if (tiles)
     gemm_q8_tile_kernel<<<(uint32_t)gemm_tile_wgs(row_tiles, n_tokens), kGemmTileThreads, 0, s>>>(
         b, cols, n_tokens, n_tiles, row_tiles, token_tiles, wsp);
-  else if (n_tiles == 1u)
-    launch_rows<1>(b, row_tiles, cols, n_tokens, n_tiles, wsp, s);
-  else if (n_tiles == 2u)
-    launch_rows<2>(b, row_tiles, cols, n_tokens, n_tiles, wsp, s);
   else
-    launch_rows<4>(b, row_tiles, cols, n_tokens, n_tiles, wsp, s);
+    switch (gemm_row_wg_tiles(n_tiles)) {
+      case 1: launch_rows<1>(b, row_tiles, cols, n_tokens, n_tiles, wsp, s); break;
+      case 2: launch_rows<2>(b, row_tiles, cols, n_tokens, n_tiles, wsp, s); break;
+      case 3: launch_rows<3>(b, row_tiles, cols, n_tokens, n_tiles, wsp, s); break;
+      default: launch_rows<4>(b, row_tiles, cols, n_tokens, n_tiles, wsp, s);
+    }
   return hipGetLastError();
 }
 

@@ -66,27 +66,30 @@ static void tile_kernel(uint32_t nb, uint32_t rows_left, uint32_t tiles_left) {
     }
 }
 
-static void rows_kernel(uint32_t nb, uint32_t rows_left) {
+static void rows_kernel(uint32_t nb, uint32_t rows_left, uint32_t pairs, uint32_t ring, uint32_t ahead) {
   const uint32_t np = nb / 2, ng = (nb + 3) / 4, n4 = (ng + 3) / 4, row_bytes = nb * 34;
   const uint64_t w_bytes = (uint64_t)rows_left * row_bytes;
   const uint32_t last_row = rows_left - 1;
-  const uint32_t chunks = 2 + 2 * n4 + 2;  // barriers and the 2 chunks staged before the first
+  // barriers, and the chunks staged before the first
+  const uint32_t chunks = (pairs == 4 ? 2 : 1) + 4 * n4 * 2 / pairs + ring - 1;
   for (uint32_t lane = 0; lane < 64; ++lane) {
     for (uint32_t k = 0; k < chunks; ++k) {
-      for (uint32_t i = 0; i < 4; ++i) {
-        const uint64_t at = (uint64_t)rows_weights(lane, last_row, row_bytes) + pair(4 * k + i, np);
+      for (uint32_t i = 0; i < pairs; ++i) {
+        const uint64_t at = (uint64_t)rows_weights(lane, last_row, row_bytes) + pair(pairs * k + i, np);
         inside(at, 16, w_bytes, "weights");
         const uint32_t r = lane / 4, unit = (lane % 4) ^ (r / 4) % 4;
-        if (4 * k + i < np && r < rows_left)
-          same(at, (uint64_t)r * row_bytes + (4 * k + i) * 68 + kUnitDword[unit] * 4, "weights");
+        if (pairs * k + i < np && r < rows_left)
+          same(at, (uint64_t)r * row_bytes + (pairs * k + i) * 68 + kUnitDword[unit] * 4, "weights");
       }
-      const uint32_t p = 4 * k + lane / 16;
-      const uint64_t e = (uint64_t)rows_dwords8(lane, last_row, row_bytes) + pair(p, np);
-      inside(e, 4, w_bytes, "dwords 8");
-      if (p < np && lane % 16 < rows_left)
-        same(e, (uint64_t)(lane % 16) * row_bytes + p * 68 + 32, "dwords 8");
+      for (uint32_t i = 0; i < pairs; i += 4) {
+        const uint32_t p = pairs * k + i + lane / 16;
+        const uint64_t e = (uint64_t)rows_dwords8(lane, last_row, row_bytes) + pair(p, np);
+        inside(e, 4, w_bytes, "dwords 8");
+        if (p < np && lane % 16 < rows_left)
+          same(e, (uint64_t)(lane % 16) * row_bytes + p * 68 + 32, "dwords 8");
+      }
     }
-    for (uint32_t g = 0; g < 4 * n4 + 5; ++g) {
+    for (uint32_t g = 0; g < 4 * n4 + 1 + ahead; ++g) {
       for (uint32_t i = 0; i < 2; ++i) {
         const uint64_t at = (uint64_t)lane * 16 + rows_quants(2 * g + i, np);
         inside(at, 16, (uint64_t)np * 1024, "quants");
@@ -117,7 +120,10 @@ int main() {
         tile_kernel(nb, rows, tiles);
       }
       std::snprintf(text, sizeof text, "16 x 16 tiles, %u blocks, %u rows", nb, rows);
-      rows_kernel(nb, rows);
+      for (uint32_t ahead : {4u, 8u}) {
+        rows_kernel(nb, rows, 4, 3, ahead);
+        rows_kernel(nb, rows, 8, 2, ahead);
+      }
     }
   }
   std::printf("ok\n");

@@ -91,21 +91,74 @@ def test_batches_that_the_gemv_takes(tmp_path):
 
 
 def test_launches_stay_within_one_grid(tmp_path):
-    """(row tiles, cols, tokens) -> 64 x 64 tiles? Sizes up to the card's memory and past it."""
+    """(rows, cols, tokens) -> 64 x 64 tiles? Sizes up to the card's memory and past it."""
     want = {
-        (448, 4096, 64): 1,
-        (448, 4096, 32): 0,                   # half a tile's tokens or fewer
-        (255, 4096, 64): 0,
-        (1, 64, 64 * (1 << 21) - 64): 1,      # 2^24 - 8 workgroups of 256
-        (1, 64, 64 * (1 << 21)): 0,           # 2^32 threads
-        (2, 64, 1 << 30): 0,
-        (2048, 64, 64 * 8191): 1,
-        (2048, 64, 64 * 8192): 0,
+        (64, 64, 64 * (1 << 21) - 64): 1,     # 2^24 - 8 workgroups of 256
+        (64, 64, 64 * (1 << 21)): 0,          # 2^32 threads
+        (128, 64, 1 << 30): 0,
+        (131072, 64, 64 * 8191): 1,
+        (131072, 64, 64 * 8192): 0,
     }
     got = _cuts(tmp_path, list(want), "gemm_plan_print")
     assert {k: g[0] for k, g in zip(want, got)} == want
-    for (row_tiles, cols, tokens), (tiles, threads, act) in zip(want, got):
-        assert not tiles or threads < 2 ** 32
-        assert act == -(-tokens // 16) * 16 * cols // 8
-    (_, _, past), = _cuts(tmp_path, [(1, 5632, 6_200_000)], "gemm_plan_print")
+    for (rows, cols, tokens), g in zip(want, got):
+        assert not g[0] or g[1] < 2 ** 32
+        assert g[2] == -(-tokens // 16) * 16 * cols // 8
+    past = _cuts(tmp_path, [(64, 5632, 6_200_000)], "gemm_plan_print")[0][2]
     assert past > 2 ** 32 - 1                 # the caller then runs the GEMV
+
+
+def test_which_matrix_core_kernel(tmp_path):
+    """(rows, cols, tokens) -> 64 x 64 tiles? us of 64 x 64 / 16 x 16, weights from HBM."""
+    want = {
+        (28672, 4096, 32): 0,     # 48.5 / 47.2
+        (28672, 4096, 33): 1,     # 50.0 / 53.7
+        (20480, 4096, 33): 0,     # 48.8 / 41
+        (20480, 4096, 64): 0,     # 50.0 / 44.3
+        (12288, 4096, 33): 0,     # 28.7 / 25.8
+        (14336, 4096, 33): 1,     # 29.1 / 33.0
+        (11264, 2048, 64): 0,     # 17.0 / 15.8
+        (11264, 2048, 65): 0,     # 20.6 / 19.0
+        (11264, 2048, 97): 1,     # 21.4 / 24.3
+        (4096, 4096, 192): 0,     # 26.6 / 23.4
+        (4096, 4096, 200): 1,     # 26.9 / 28.6
+        (5120, 5120, 129): 0,     # 31.6 / 28.4
+        (5120, 5120, 160): 1,     # 32.4 / 34.7
+        (8192, 8192, 129): 0,     # 74.1 / 66.8
+        (8192, 8192, 192): 1,     # 76.1 / 80.8
+        (4096, 14336, 200): 1,    # 78.4 / 83.6
+        (4096, 14336, 320): 0,    # 123.4 / 100.7
+        (4096, 14336, 512): 1,    # 129.8 / 159.3
+        (4480, 832, 256): 1,      # 13.8 / 16.1: 26 blocks run as 32
+        (17408, 4096, 65): 0,     # 57.5 / 48.5
+        (6144, 4096, 384): 1,     # 47.9 / 57.0
+    }
+    got = _cuts(tmp_path, list(want), "gemm_plan_print")
+    assert {k: g[0] for k, g in zip(want, got)} == want
+
+
+def test_cut_of_the_16x16_kernel(tmp_path):
+    """(rows, cols, tokens) -> token tiles a workgroup, wide chunks, groups ahead, spare LDS."""
+    want = {
+        (4096, 4096, 16): (1, 0, 4, 0),
+        (4096, 14336, 16): (1, 0, 8, 0),          # 26.4 us, 4 ahead 30.7
+        (8192, 8192, 8): (1, 0, 8, 0),            # 21.4, 23.5
+        (11264, 8192, 16): (1, 0, 4, 0),
+        (14336, 4096, 16): (1, 0, 4, 0),          # 23.0, three a CU 27.5
+        (22528, 4096, 16): (1, 0, 4, 35840),      # 30.6, eight a CU 35.5
+        (4096, 4096, 32): (2, 0, 4, 0),
+        (4096, 14336, 32): (2, 1, 8, 0),          # 28.3, 33.6
+        (20480, 4096, 32): (2, 0, 4, 0),          # 35.4, three a CU 37.2
+        (28672, 8192, 32): (2, 1, 8, 35840),      # 82.2, 86.0
+        (4096, 4096, 33): (3, 1, 4, 0),
+        (4096, 14336, 33): (3, 1, 8, 0),
+        (17408, 4096, 33): (3, 1, 4, 35840),      # 35.9, 38.3
+        (1024, 8192, 192): (4, 1, 4, 0),          # 20.3, 8 ahead 20.5
+        (4096, 14336, 64): (4, 1, 8, 0),          # 30.5, 35.8
+        (4096, 14336, 65): (3, 1, 4, 0),
+        (4096, 14336, 128): (4, 1, 4, 0),
+        (4096, 14336, 129): (3, 1, 4, 0),         # 9 tiles: 3 groups of 3
+        (4096, 14336, 145): (4, 1, 4, 0),
+    }
+    got = _cuts(tmp_path, list(want), "gemm_plan_print")
+    assert {k: tuple(g[3:]) for k, g in zip(want, got)} == want

@@ -59,6 +59,9 @@ def _gemv(w, rows, cols, x):
     (3073, 1024, 8), (3088, 2048, 9), (1569, 1024, 16), (1456, 3072, 17), (801, 1024, 31),
     (784, 1024, 32), (736, 4096, 33), (513, 1024, 48), (399, 2048, 63), (385, 1024, 64),
     (400, 3072, 65), (129, 2048, 200), (4097, 1024, 8), (17, 1024, 770),
+    # one to four token tiles a workgroup with 8 groups loaded ahead, an odd number of runs
+    (3100, 8704, 16), (1600, 8704, 32), (3090, 8704, 40), (3090, 8704, 64),
+    (16400, 1024, 8), (20500, 1024, 20), (16400, 1024, 40),  # with spare LDS
 ])
 def test_matches_oracle_and_gemv(rows, cols, n_tokens):
     rng = np.random.default_rng(rows * 131 + cols + n_tokens)
@@ -119,14 +122,21 @@ def test_non_finite_and_extreme_inputs(rows):
 
 
 @pytest.mark.parametrize("rows,cols,n_tokens", [
-    ([16385], 1024, 48),              # the fewest tokens, one row past the last row tile
-    ([8200], 2048, 65),               # one token past a tile
+    ([16385], 1024, 48),              # 257 workgroups: 16 x 16 tiles
+    ([28673], 1024, 48),              # 449, one row past the last row tile: 32 x 32
+    ([28673], 1024, 33),              # the fewest tokens
+    ([28673], 1024, 32),              # and one fewer: 16 x 16 tiles
+    ([12289], 1024, 33),              # up to 256, past 192
+    ([8200], 2048, 65),               # one token past a tile: 16 x 16 tiles,
+    ([14400], 1024, 65),              # and of more rows 32 x 32
     ([4032, 64, 1], 1024, 256),       # three matrices, whole tiles and one row
-    ([4100], 3072, 250),
+    ([5056, 64, 1], 1024, 256),
+    ([4100], 3072, 250), ([5200], 3072, 250),
 ])
-def test_large_launches_in_32x32_tiles(rows, cols, n_tokens):
-    """Launches of 256 workgroups of 64 x 64 outputs or more, non-finite scales among the
-    weights and activations: every output is the oracle's."""
+def test_large_launches(rows, cols, n_tokens):
+    """Launches of 256 workgroups of 64 x 64 outputs or more, on either side of the line
+    between the two kernels, non-finite scales among the weights and activations: every
+    output is the oracle's."""
     rng = np.random.default_rng(cols + n_tokens)
     ws = [_weights(rng, r, cols, special=True) for r in rows]
     x = (rng.standard_normal((n_tokens, cols)) *
@@ -145,7 +155,8 @@ def test_large_launches_in_32x32_tiles(rows, cols, n_tokens):
     (16400, 320, 70, 4),   # 32 x 32 tiles, an odd number of pairs
     # the same widths in launches large enough for the matrix cores
     (3080, 64, 8, 0), (1569, 192, 16, 4), (1456, 448, 17, 8), (752, 576, 33, 12),
-    (2070, 5632, 11, 0),
+    (2070, 5632, 11, 0), (3090, 8256, 16, 4), (3090, 8256, 40, 8), (16400, 320, 9, 4),
+    (20500, 320, 20, 0),
     # 32 x 32 tiles of one and two chunks of blocks, whole and not
     (8200, 64, 70, 12), (8200, 128, 70, 8), (8200, 192, 70, 0), (8200, 256, 70, 4),
 ])
