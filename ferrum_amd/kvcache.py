@@ -22,6 +22,7 @@ from . import _lib
 from .errors import check
 
 _torch_loaded = None
+_Tensor = None  # torch.Tensor
 _raw_stream = None  # torch's (current raw stream of a device, current device) functions
 
 
@@ -29,13 +30,14 @@ def _torch():
     """torch, imported by the first device call: the host-only surface neither needs it nor
     waits for it (2 s), and a device call without it is its ImportError. A global read
     afterwards, as an import statement is 0.2 us in every call."""
-    global _torch_loaded, _raw_stream
+    global _torch_loaded, _Tensor, _raw_stream
     if _torch_loaded is None:
         import torch
         get = getattr(torch._C, "_cuda_getCurrentRawStream", None)
         device = getattr(torch._C, "_cuda_getDevice", None)
         if get is not None and device is not None:
             _raw_stream = get, device
+        _Tensor = torch.Tensor
         _torch_loaded = torch
     return _torch_loaded
 
@@ -177,13 +179,23 @@ def _stream_ptr(stream) -> int:
 
 
 def _dev(t, dtype, name):
-    if not isinstance(t, _torch_loaded.Tensor) or not t.is_cuda:
+    if not isinstance(t, _Tensor) or not t.is_cuda:
         raise TypeError(f"{name} must be a device tensor")
     if t.dtype != dtype:
         raise TypeError(f"{name} must be {dtype}, got {t.dtype}")
     if not t.is_contiguous():
         raise ValueError(f"{name} must be contiguous")
     return t.data_ptr()
+
+
+def _dev_any(t, dtype, name):
+    if not isinstance(t, _Tensor) or not t.is_cuda:
+        raise TypeError(f"{name} must be a device tensor")
+    if t.dtype != dtype:
+        raise TypeError(f"{name} must be {dtype}, got {t.dtype}")
+    if not t.is_contiguous():
+        raise ValueError(f"{name} must be contiguous")
+    return t.data_ptr(), t.numel()
 
 
 class PagedKvPool:

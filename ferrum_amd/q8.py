@@ -17,9 +17,9 @@ from __future__ import annotations
 
 import ctypes
 
-from . import _lib, kvcache
+from . import _lib
 from .errors import check
-from .kvcache import _stream_ptr, _torch
+from .kvcache import _dev_any, _stream_ptr, _torch
 
 __all__ = ["Q8_0_BLOCK", "Q8_0_BLOCK_BYTES", "gemv_q8_0", "gemm_q8_0", "gemm_q8_0_multi",
            "gemm_q8_0_batched", "gemm_q8_0_batched_workspace_bytes", "q8_0_row_bytes"]
@@ -31,16 +31,6 @@ Q8_0_BLOCK_BYTES = 34
 def q8_0_row_bytes(cols: int) -> int:
     """Bytes of one Q8_0 weight row (pack.rs:37-44)."""
     return cols // Q8_0_BLOCK * Q8_0_BLOCK_BYTES
-
-
-def _dev_any(t, dtype, name):
-    if not isinstance(t, kvcache._torch_loaded.Tensor) or not t.is_cuda:
-        raise TypeError(f"{name} must be a device tensor")
-    if t.dtype != dtype:
-        raise TypeError(f"{name} must be {dtype}, got {t.dtype}")
-    if not t.is_contiguous():
-        raise ValueError(f"{name} must be contiguous")
-    return t.data_ptr(), t.numel()
 
 
 def gemv_q8_0(w, rows: int, cols: int, x, y, stream=None) -> None:

@@ -49,10 +49,11 @@ def test_stream_handle_without_torch_private_functions(monkeypatch):
     from ferrum_amd import kvcache
     stream = types.SimpleNamespace(cuda_stream=1234)
     cuda = types.SimpleNamespace(is_initialized=lambda: True, current_stream=lambda: stream)
-    fake = types.SimpleNamespace(_C=types.SimpleNamespace(), cuda=cuda)
+    fake = types.SimpleNamespace(_C=types.SimpleNamespace(), cuda=cuda, Tensor=object)
     monkeypatch.setitem(sys.modules, "torch", fake)
     monkeypatch.setattr(kvcache, "_torch_loaded", None)
     monkeypatch.setattr(kvcache, "_raw_stream", None)
+    monkeypatch.setattr(kvcache, "_Tensor", None)
     assert kvcache._stream_ptr(None) == 1234
     fake._C._cuda_getCurrentRawStream = lambda device: 100 + device
     fake._C._cuda_getDevice = lambda: 3
