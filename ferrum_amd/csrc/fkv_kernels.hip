@@ -378,8 +378,9 @@ __device__ __forceinline__ int64_t drop_repeated_slot(int64_t sl) {
 // j + 32, j + 48 of 4 consecutive tokens; for each segment of the window (a maximal run
 // of consecutive slots inside one 4-aligned token group) it is stored whole when the
 // segment is the whole group and by single bytes otherwise.
-// Measured with 8 KV heads of 128 dims, 8,192 tokens (84 MB): 30.6 -> 25.5 us, 3.3 TB/s;
-// 24,000 tokens 54.2 -> 52.7 (4.7 TB/s).
+// Measured with 8 KV heads of 128 dims, 8,192 tokens (84 MB): 30.6 -> 24.9 us, 3.4 TB/s;
+// 24,000 tokens 54.2 -> 49.4 (5.0 TB/s). (Scales stored before the barrier, and repeated
+// slots looked for before the rows are asked for: 27.1 and 52.2.)
 // A slot named twice in a window goes to the last of its tokens (drop_repeated_slot): its
 // scales and quants are stored by different waves.
 template <int D>
@@ -394,7 +395,7 @@ __global__ void __launch_bounds__(256) append_q8_tile_kernel(Geom g, uint32_t la
   constexpr uint32_t kUnits = D / 16;        // K units of a token
   static_assert(kHpw * kRuns == 16, "head_dim 64 or 128");
   constexpr uint32_t cpr = D / 32;
-  __shared__ int64_t s_slot[16];
+  __shared__ int64_t s_slot[16], s_keep[16];  // and without the repeated ones
   // rows of 16 tokens' K units and of a token's V quants, padded so that the strided
   // side of each transpose meets distinct banks
   __shared__ __align__(16) uint8_t s_k[kHpw][kUnits][16 * 16 + 16];
@@ -414,12 +415,11 @@ __global__ void __launch_bounds__(256) append_q8_tile_kernel(Geom g, uint32_t la
       raise_fault(g.fault, kFaultSlot);
       sl = -1;
     }
-    s_slot[threadIdx.x] = drop_repeated_slot(sl);
+    s_slot[threadIdx.x] = sl;
   }
   __syncthreads();
 
-  const int64_t slot = s_slot[o];
-  const bool live = slot >= 0 && h < g.n_kv_heads;
+  const bool live = s_slot[o] >= 0 && h < g.n_kv_heads;
   float x[2][8] = {};
   if (live) {
     const uint64_t at = (((uint64_t)win * 16u + o) * g.n_kv_heads + h) * D + r * 8u;
@@ -431,6 +431,9 @@ __global__ void __launch_bounds__(256) append_q8_tile_kernel(Geom g, uint32_t la
       x[kv][4] = b.x; x[kv][5] = b.y; x[kv][6] = b.z; x[kv][7] = b.w;
     }
   }
+  // (while the rows are on their way)
+  if (threadIdx.x < 16) s_keep[threadIdx.x] = drop_repeated_slot(s_slot[threadIdx.x]);
+  uint32_t sc[2];
 #pragma unroll
   for (int kv = 0; kv < 2; kv++) {
     float amax = 0.0f;
@@ -444,19 +447,7 @@ __global__ void __launch_bounds__(256) append_q8_tile_kernel(Geom g, uint32_t la
 #pragma unroll
     for (int j = 0; j < 8; j++)
       q[j / 4] |= ((uint32_t)q8_quant(x[kv][j], id) & 0xffu) << (8 * (j % 4));
-    if (live && r % 4u == 0u) {
-      const uint32_t sc = encode_f16(d, g.rounding);
-      const uint64_t blk = (uint64_t)slot / B;
-      const uint32_t off = (uint32_t)((uint64_t)slot % B);
-      ((uint16_t*)(tile_ptr(g, blk, layer, kv, h) + (uint64_t)B * D))[off * cpr + r / 4u] = (uint16_t)sc;
-      // A scale of 512 or more marks the block (attention over it takes the exact
-      // instance); one past the binary16 range is stored as +-inf, as the reference's
-      // encoder stores it, and flagged.
-      if (q8_wide_scale(sc)) {
-        mark_block(g, blk);
-        if ((sc & 0x7c00u) == 0x7c00u) raise_fault(g.fault, kFaultRange);
-      }
-    }
+    sc[kv] = encode_f16(d, g.rounding);
     if (kv == 0) {  // unit (pair r / 8, run r % 4), half of the block
       *(uint2*)&s_k[hl][r / 8u * 4u + r % 4u][o * 16u + (r / 4u) % 2u * 8u] = make_uint2(q[0], q[1]);
     } else {
@@ -467,10 +458,27 @@ __global__ void __launch_bounds__(256) append_q8_tile_kernel(Geom g, uint32_t la
   }
   __syncthreads();
 
+  const int64_t slot = s_keep[o];
+  if (slot >= 0 && h < g.n_kv_heads && r % 4u == 0u) {
+    const uint64_t blk = (uint64_t)slot / B;
+    const uint32_t off = (uint32_t)((uint64_t)slot % B);
+#pragma unroll
+    for (int kv = 0; kv < 2; kv++) {
+      ((uint16_t*)(tile_ptr(g, blk, layer, kv, h) + (uint64_t)B * D))[off * cpr + r / 4u] = (uint16_t)sc[kv];
+      // A scale of 512 or more marks the block (attention over it takes the exact
+      // instance); one past the binary16 range is stored as +-inf, as the reference's
+      // encoder stores it, and flagged.
+      if (q8_wide_scale(sc[kv])) {
+        mark_block(g, blk);
+        if ((sc[kv] & 0x7c00u) == 0x7c00u) raise_fault(g.fault, kFaultRange);
+      }
+    }
+  }
+
   const uint32_t t = threadIdx.x % 128u;  // 128 units of K (waves 0, 1) and of V (2, 3)
   if (threadIdx.x < 128u) {
     const uint32_t e = t % 16u, un = (t / 16u) % kUnits, uh = t / (16u * kUnits);
-    const int64_t sl = s_slot[e];
+    const int64_t sl = s_keep[e];
     if (sl < 0 || hg * kHpw + uh >= g.n_kv_heads) return;
     uint8_t* tile = tile_ptr(g, (uint64_t)sl / B, layer, 0, hg * kHpw + uh);
     *(uint4*)(tile + q8_quant_offset(0, (uint32_t)((uint64_t)sl % B), un / 4u * 64u + un % 4u * 8u, D)) =
@@ -484,10 +492,10 @@ __global__ void __launch_bounds__(256) append_q8_tile_kernel(Geom g, uint32_t la
   const uint32_t hv = hg * kHpw + vh;
   if (hv >= g.n_kv_heads) return;
   for (uint32_t e0 = 4u * part; e0 < 4u * part + 4u; e0++) {
-    const int64_t s0 = s_slot[e0];
-    if (s0 < 0 || (e0 > 0 && s0 % 4 != 0 && s_slot[e0 - 1] == s0 - 1)) continue;
+    const int64_t s0 = s_keep[e0];
+    if (s0 < 0 || (e0 > 0 && s0 % 4 != 0 && s_keep[e0 - 1] == s0 - 1)) continue;
     uint32_t len = 1;
-    while (e0 + len < 16u && (s0 + len) % 4 != 0 && s_slot[e0 + len] == s0 + (int64_t)len) len++;
+    while (e0 + len < 16u && (s0 + len) % 4 != 0 && s_keep[e0 + len] == s0 + (int64_t)len) len++;
     const uint32_t off = (uint32_t)((uint64_t)s0 % B);
     uint8_t* unit = tile_ptr(g, (uint64_t)s0 / B, layer, 1, hv) +
                     (q8_quant_offset(1, off, vi * 64u + j, D) & ~(uint64_t)15);
