@@ -1066,9 +1066,10 @@ def run_q8gemv(args, torch, fa, lib, dev):
     n_launch = K * len(calls)
     value = step_bytes * K / wall / 1e9
     achieved = step_bytes / len(calls) / (region_ms * 1e-3 / n_launch) / 1e9
-    kname = "gemv_q8_kernel<%d>" % (4 if T >= 3 else T)
+    kname = "gemv_q8_kernel"
     if args.gemm_batched and T >= 8:
-        kname = "q8_act_kernel + gemm_q8_mfma_kernel (fkv_gemm_q8_0_batched)"
+        kname = ("q8_act_tile_kernel + gemm_q8_tile_kernel or gemm_q8_rows_kernel "
+                 "(fkv_gemm_q8_0_batched)")
     res = {
         "metric": "Q8_0 weight GEMV HBM GB/s (Llama-3-8B decode projections), 1xMI355X",
         "value": round(value, 2),
@@ -1219,9 +1220,9 @@ def run_layer(args, torch, fa, lib, dev):
         "us_per_layer": round(region_ms * 1e3 / (K * L), 2),
         "bytes_per_step": {"weights": int(w_bytes), "kv": int(np.mean(kv) * L),
                            "activations": int(act * L)},
-        "roofline": {"bound": "hbm", "kernel": "whole layer (q8_act_kernel + "
-                     "gemm_q8_mfma_kernel, attn_mfma_kernel + attn_combine_kernel, "
-                     "q8_act_kernel + gemm_q8_mfma_kernel)",
+        "roofline": {"bound": "hbm", "kernel": "whole layer (q8_act_tile_kernel + "
+                     "gemm_q8_rows_kernel, attn_mfma_kernel + attn_combine_kernel, "
+                     "q8_act_tile_kernel + gemm_q8_rows_kernel)",
                      "achieved": round(sum(step_bytes) / K / (region_ms * 1e-3 / K) / 1e9, 2),
                      "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(sum(step_bytes) / (region_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),

@@ -1,6 +1,6 @@
 // Batched Q8_0 GEMM on the matrix cores of gfx950, for batches of activation rows (a
-// decode step's sequences, a prefill chunk): the GEMV reads every weight once per 4
-// tokens. The activation is quantized once, into a workspace; then one of two kernels,
+// decode step's sequences, a prefill chunk): the GEMV reads every weight once per 1
+// to 4 tokens. The activation is quantized once, into a workspace; then one of two kernels,
 // 32 x 32 tiles first.
 //
 // The result is the GEMV's (fkv_gemv.hip) bit for bit: per output, starting from +0 and
@@ -19,10 +19,12 @@
 //   whose second to fourth terms are zero: the product of two binary16 values is exact in
 //   f32, Inf and NaN included. (The f32 form of the same outer product held up the VALU:
 //   780 against 953 TFLOP/s in a register-only loop of these instructions.)
-// Measured at 512 tokens on Llama-3-8B's projections (one box, with the quantizer; before:
-// 16 x 16 tiles, one a wave, on the four-instruction epilogue): q/k/v 85.7 -> 55.0 us,
-// attn_output 55.1 -> 40.4, gate/up 344 -> 249 (483 TFLOP/s), down 171 -> 125. Three waves
-// a SIMD take 217 cycles a block together; the clock is 1.6-1.8 GHz under that load.
+// Measured at 512 tokens on Llama-3-8B's projections (the 32 x 32 kernel alone, from a kernel
+// trace; distinct weights each call): q/k/v 54.8 us, attn_output 39.5, gate/up 218 (551
+// TFLOP/s), down 130; the four calls with their quantizers 443 us, where 16 x 16 tiles, one a
+// wave, on the four-instruction epilogue took 642. Three waves a SIMD take 223 cycles a block
+// together, 94% of them issue VALU instructions, and the clock is about 1.9 GHz under that
+// load.
 #include "fkv_device.h"
 #include "fkv_gemm_at.h"
 #include "fkv_gemm_plan.h"
@@ -336,10 +338,11 @@ __global__ __launch_bounds__(256, 2) void gemm_q8_tile_kernel(const GemvBatch ba
 // The same sums (integer dots from v_mfma_i32_16x16x32_i8, four blocks' products of scales
 // from one v_mfma_f32_16x16x4_4b_f16, three VALU instructions per output and block), for
 // launches that would leave CUs without work in 64 x 64 tiles, or most of their tokens
-// unused. The ordered sum makes a row tile one chain, a wave takes about 80-90 cycles a
-// block, and a CU has few waves: the chain bounds launches of few rows (down of
-// Llama-3-8B, 448 blocks: 25 us at 16 tokens where the weights alone stream in 10), and
-// what matters is that nothing else is waited for. A further wave streams the weights
+// unused. The ordered sum makes a row tile one chain, a wave takes 95 cycles a block at best
+// (one row tile, weights from cache) and about 120 with a CU's weights from HBM, and a CU has
+// few waves: the chain bounds launches of few rows (down of Llama-3-8B, 448 blocks: 23 us at
+// 16 tokens where the weights alone stream in 10), and what matters is that nothing else is
+// waited for. A further wave streams the weights
 // through a ring of chunks in LDS by direct loads; the computing waves load the
 // activation, which the L2 holds, four groups of blocks ahead into registers. Loads retire
 // in order, so with the weight loads in the computing waves each activation load would

@@ -80,8 +80,11 @@ def gemm_q8_0_batched_workspace_bytes(cols: int, n_tokens: int) -> int:
 def gemm_q8_0_batched(ws, rows, cols: int, x, n_tokens: int, ys, workspace=None,
                       stream=None) -> None:
     """gemm_q8_0_multi on the matrix cores for batches (n_tokens >= 8, cols a multiple of
-    64, 4-byte aligned weights; otherwise the GEMV), bit-identical. `workspace`: a
-    device uint8 tensor of gemm_q8_0_batched_workspace_bytes (allocated here when None)."""
+    64, 4-byte aligned weights, more than the GEMV runs at once; otherwise the GEMV),
+    bit-identical. `workspace`: a device uint8 tensor of gemm_q8_0_batched_workspace_bytes
+    (allocated here when None). A smaller one, or one off 16 bytes, is an InvalidRequest where
+    cols is a multiple of 1024 and every weight 16-byte aligned, and runs the GEMV elsewhere,
+    which is many times slower for large batches."""
     torch = _torch()
     n = len(ws)
     if len(rows) != n or len(ys) != n:

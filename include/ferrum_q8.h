@@ -76,7 +76,7 @@ int32_t fkv_gemm_q8_0_multi(uint32_t n_mats, const void* const* w, const uint64_
 /* fkv_gemm_q8_0_multi for batches of activation rows (a decode step's sequences, a
  * prefill chunk) on the matrix cores, with the same results bit for bit. No counterpart
  * in the reference, which loops over tokens (scalar.rs:98-116); the entry points above
- * read every weight once per 4 tokens. Here each activation row is quantized once into
+ * read every weight once per 1 to 4 tokens. Here each activation row is quantized once into
  * `workspace`, and i8 MFMAs give a 32-value block's exact integer dots for 16 x 16 or
  * 32 x 32 outputs; each output then accumulates f32(sumi) * (w_scale * x_scale) block by
  * block in order, as dot_q8_row_q8_act does.
@@ -87,8 +87,8 @@ int32_t fkv_gemm_q8_0_multi(uint32_t n_mats, const void* const* w, const uint64_
  * workspace must hold fkv_gemm_q8_0_batched_workspace_size() bytes and be 16-byte aligned:
  * where cols is a multiple of 1024 and every w 16-byte aligned one that is not is
  * FKV_ERR_INVALID "gemm workspace too small" / "gemm workspace must be 16-byte aligned",
- * elsewhere (NULL included) the call runs the GEMV. The workspace needs no
- * initialisation; calls that share one must not overlap. */
+ * elsewhere (NULL included) the call runs the GEMV, many times slower for large batches.
+ * The workspace needs no initialisation; calls that share one must not overlap. */
 int32_t fkv_gemm_q8_0_batched_workspace_size(uint64_t cols, uint64_t n_tokens,
                                              uint64_t* bytes_out);
 int32_t fkv_gemm_q8_0_batched(uint32_t n_mats, const void* const* w, const uint64_t* w_len,

@@ -223,6 +223,46 @@ def test_workspace_size_and_rejection():
     assert np.all(y.cpu().numpy() == 5.0)
 
 
+@pytest.mark.parametrize("cols,refused", [(576, False), (1024, True)])
+def test_workspaces_through_the_c_abi(cols, refused):
+    """NULL, too small and misaligned: refused where columns are a multiple of 1024, a GEMV
+    elsewhere (the workspace untouched), and the matrix cores with one that does."""
+    import ctypes
+    import torch
+    from ferrum_amd import _lib
+    lib = _lib.load()
+    rows, n_tokens = 1600, 30
+    rng = np.random.default_rng(cols)
+    w = _weights(rng, rows, cols)
+    x = rng.standard_normal((n_tokens, cols)).astype(np.float32)
+    want = ref.q8_gemm(w, rows, cols, x)
+    wd, xd = _dev(w), _dev(x)
+    need = ctypes.c_uint64()
+    assert lib.fkv_gemm_q8_0_batched_workspace_size(cols, n_tokens, ctypes.byref(need)) == 0
+    need = need.value
+    ws = torch.full((need + 16,), 0x5a, dtype=torch.uint8, device="cuda")
+    for ptr, size, error in [(None, 0, "too small"), (None, need, "too small"),
+                             (ws.data_ptr(), need - 1, "too small"),
+                             (ws.data_ptr() + 4, need, "must be 16-byte aligned"),
+                             (ws.data_ptr(), need, None)]:
+        y = torch.full((n_tokens, rows), 5.0, dtype=torch.float32, device="cuda")
+        one = lambda t, v: (t * 1)(v)
+        st = lib.fkv_gemm_q8_0_batched(
+            1, one(ctypes.c_void_p, wd.data_ptr()), one(ctypes.c_uint64, wd.numel()),
+            one(ctypes.c_uint64, rows), cols, xd.data_ptr(), xd.numel(), n_tokens,
+            one(ctypes.c_void_p, y.data_ptr()), one(ctypes.c_uint64, y.numel()), ptr, size,
+            torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        if error and refused:
+            assert st == _lib.FKV_ERR_INVALID
+            assert lib.fkv_last_error().decode() == "gemm workspace " + error
+            assert bool((y == 5.0).all())
+        else:
+            assert st == 0
+            _same(y.cpu().numpy(), want)
+        assert bool((ws != 0x5a).any()) == (error is None)
+
+
 @pytest.mark.parametrize("case", range(20))
 def test_randomized_batches_against_oracle_and_gemv(case):
     """Seeded random launches: 1 to 4 matrices (an empty one possible) sharing an
