@@ -132,7 +132,7 @@ struct Chunk {
   uint32_t xs[2][2][2][32];    // [pair][token half][block][token]
 };
 
-// A workgroup: 64 weight rows x 64 tokens, a wave 32 x 32; 3 workgroups a CU (157 VGPRs,
+// A workgroup: 64 weight rows x 64 tokens, a wave 32 x 32; 3 workgroups a CU (154 VGPRs,
 // 52.5 KiB of LDS). Everything is staged by loads straight into LDS, two to three chunks
 // ahead (three buffers), so that no wave spends registers or instructions on it. (Weights
 // through registers with the repacking done by the computing waves: gate/up 285 us; by two
@@ -342,11 +342,10 @@ __global__ __launch_bounds__(256, 2) void gemm_q8_tile_kernel(const GemvBatch ba
 // (one row tile, weights from cache) and about 120 with a CU's weights from HBM, and a CU has
 // few waves: the chain bounds launches of few rows (down of Llama-3-8B, 448 blocks: 23 us at
 // 16 tokens where the weights alone stream in 10), and what matters is that nothing else is
-// waited for. A further wave streams the weights
-// through a ring of chunks in LDS by direct loads; the computing waves load the
-// activation, which the L2 holds, four groups of blocks ahead into registers. Loads retire
-// in order, so with the weight loads in the computing waves each activation load would
-// wait for HBM. Against the kernel before (one variant with and one without such a wave,
+// waited for. A further wave streams the weights through a ring of chunks in LDS by direct
+// loads; the computing waves load the activation, which the L2 holds, four or eight groups of
+// blocks ahead into registers. Loads retire in order, so with the weight loads in the
+// computing waves each activation load would wait for HBM. Against the kernel before (one variant with and one without such a wave,
 // weights through registers, four VALU instructions), us with weights from HBM, 16 tokens:
 // q/k/v 14.3 -> 12.1, attn_output 12.9 -> 11.4, gate/up 40.8 -> 40.0, down 29.3 -> 26.4; 64
 // tokens: 19.0 -> 15.9, 14.5 -> 13.3, gate/up in 64 x 64 tiles, 35.0 -> 30.1.
