@@ -1,5 +1,5 @@
 /* Exhaustive CPU check of two f32 identities the Q8_0 GEMV kernel relies on
- * (ferrum_amd/csrc/fkv_gemv.hip: div127, round_away). Both use only IEEE f32
+ * (ferrum_amd/csrc/fkv_q8_act.h: div127, round_away). Both use only IEEE f32
  * multiply, add, fma and trunc, which the GPU computes identically:
  *   div127(a) = fma(fma(-a*c, 127, a), c, a*c), c = RN(1/127)  == a / 127
  *       for every a in [0, +Inf) (and +Inf mapped to +Inf separately);
