@@ -1,4 +1,4 @@
-"""The Q8_0 products's short forms of d = amax / 127 and of Rust's round are the
+"""The Q8_0 products' short forms of d = amax / 127 and of Rust's round are the
 reference's operations bit for bit (ferrum_amd/csrc/fkv_q8_act.h: div127,
 round_away): checked here over every f32 input on the CPU, where IEEE f32 multiply,
 add, fma and trunc give what the GPU's v_mul/v_add/v_fma/v_trunc give."""

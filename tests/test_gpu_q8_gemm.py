@@ -98,7 +98,7 @@ def test_matches_oracle(rows, cols, n_tokens):
 
 @pytest.mark.parametrize("rows,cols,n_tokens", [
     (8176, 64, 3), (8177, 64, 3),      # 511 and 512 workgroups of 16 rows: 2 and 4 tokens each
-    (11984, 96, 8), (12000, 96, 7),    # 1,498 and 1,500 workgroups of 4 tokens
+    (11984, 96, 8), (12000, 96, 7),    # 1,498 and 1,500 workgroups of 4 tokens: 4
     (5584, 96, 8), (5600, 96, 7),      # 698 (2 tokens each) and 700 of them
     (6144, 64, 10),                    # 1,152, 5 rounds of the CUs against 8: 2 tokens
     (800, 4128, 117), (800, 4128, 114),  # past 4,096 columns 1,500 and 1,450: 4 and 2
